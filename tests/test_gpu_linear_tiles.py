@@ -1,0 +1,104 @@
+"""Edges of the fp32-activation reader's tile kernels (uq_frontier.hip) against the
+CPU oracle: ragged tiles of 16 rows, columns that fill no whole step (128 or 256
+values), fewer steps than a workgroup has waves, many tiles per workgroup, groups
+of 256 values whose range exceeds the integer digits, infinite block scales, and
+both launch forms of a job table.
+
+Outputs are the exact double sum rounded to f32 once, so the bound is 1 ulp (a
+double sum a few 2^-53 off may round the other way)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as O
+import uq
+from test_gpu_linear import ulps
+
+pytestmark = pytest.mark.gpu
+
+TILE_KINDS = [k for k in uq.LINEAR_KINDS if k not in (uq.KIND_F32, uq.KIND_BF16)]
+BLOCK32 = (uq.KIND_Q8_0, uq.KIND_IQ4_NL)
+
+
+def check(kind, n, m, x, seed):
+    raw = uq.synth_quant(kind, seed, m, n)
+    y = uq.linear(uq.Weight(kind, n, m, raw), x)
+    ref = O.linear(kind, raw, n, m, x)
+    assert ulps(y, ref).max() <= 1, (kind, n, m)
+    return y
+
+
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 4097])
+def test_ragged_rows(gpu, kind, m):
+    check(kind, 512, m, uq.synth_normal(m, 512), 0x711 + kind)
+
+
+@pytest.mark.parametrize("kind,n", [(k, n) for k in BLOCK32 for n in (32, 96, 160, 288, 1056, 2528)] +
+                         [(k, n) for k in TILE_KINDS for n in (256, 768, 2304, 16384)])
+def test_columns(gpu, kind, n):
+    check(kind, n, 50, uq.synth_normal(n, n), 0xC01 + kind)
+
+
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("n", [256, 1280])
+def test_many_tiles_per_workgroup(gpu, kind, n):
+    # 20011 rows = 1251 tiles: several tiles for every workgroup of 256 CUs
+    check(kind, n, 20011, uq.synth_normal(n + 1, n), 0x3A9 + kind)
+
+
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("groups", [(0,), (1, 4), (0, 1, 2, 3, 4)])
+def test_wide_groups(gpu, kind, groups):
+    """Groups of 256 values whose smallest value lies more than 2^38 below the
+    largest run in double, the others beside them on the digits."""
+    n = 1280
+    x = uq.synth_normal(kind, n)
+    for g in groups:
+        x[256 * g + 7] = np.float32(1e-20)
+        x[256 * g + 200] = np.float32(-3e-39)  # denormal
+    check(kind, n, 100, x, 0x51D + kind)
+    x[3] = np.float32(2e30)  # and a value that swamps its own group
+    check(kind, n, 100, x, 0x51E + kind)
+
+
+@pytest.mark.parametrize("kind,offset", [(uq.KIND_Q8_0, 0), (uq.KIND_IQ4_NL, 0), (uq.KIND_IQ4_XS, 0),
+                                         (uq.KIND_IQ3_XXS, 0), (uq.KIND_Q6_K, 208)])
+def test_infinite_scale(gpu, kind, offset):
+    """A row with an infinite block scale is not finite; the rows of its tile and
+    the other tiles keep their values."""
+    n, m = 1024, 40
+    raw = uq.synth_quant(kind, 0x1F + kind, m, n)
+    rb = uq.row_bytes(kind, n)
+    raw[20 * rb + offset], raw[20 * rb + offset + 1] = 0x00, 0x7C
+    x = uq.synth_normal(kind + 9, n)
+    w = uq.Weight(kind, n, m, raw)
+    L = uq.lib()
+    dx, dy = ctypes.c_void_p(), ctypes.c_void_p()
+    assert L.uq_dev_alloc(4 * n, ctypes.byref(dx)) == 0 and L.uq_dev_alloc(4 * m, ctypes.byref(dy)) == 0
+    try:
+        assert L.uq_memcpy_h2d(dx, x.ctypes.data, 4 * n) == 0
+        assert L.uq_linear_dev(w.handle, dx, dy, None) == 0
+        y = np.empty(m, np.float32)
+        assert L.uq_memcpy_d2h(y.ctypes.data, dy, 4 * m) == 0
+    finally:
+        L.uq_dev_free(dx)
+        L.uq_dev_free(dy)
+    ref = O.linear(kind, raw, n, m, x)
+    assert not np.isfinite(y[20]) and not np.isfinite(ref[20])
+    rest = np.arange(m) != 20
+    assert ulps(y[rest], ref[rest]).max() <= 1
+
+
+@pytest.mark.parametrize("sizes", [[40] * 12, [5000] + [3] * 30, [1, 16, 17, 700]])
+def test_job_table_forms_equal_single_calls(gpu, sizes):
+    """Tables of similar jobs (a grid row per job) and of very unequal ones (starts
+    searched) give the bits of the single calls."""
+    pairs = []
+    for i, m in enumerate(sizes):
+        kind = uq.LINEAR_KINDS[i % len(uq.LINEAR_KINDS)]
+        n = (512, 1024)[i % 2]
+        pairs.append((uq.Weight(kind, n, m, uq.synth_quant(kind, i, m, n)), uq.synth_normal(i, n)))
+    for (w, x), y in zip(pairs, uq.linear_batch(pairs)):
+        assert np.array_equal(y.view(np.uint32), uq.linear(w, x).view(np.uint32))

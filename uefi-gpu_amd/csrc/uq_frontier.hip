@@ -11,17 +11,29 @@
 // Arithmetic. Every decoded weight of these kinds is an integer code times an
 // f32 block scale that is itself an exact product (fp16 d times a small
 // integer, or a power-of-two fraction of one), so sum_i w_i x_i equals
-// sum over scale groups of scale * sum(code * x) exactly. The kernels form
-// each code * x in double (exact), sum a scale group in double, multiply by
-// the exact scale in double, add the groups of a lane in unit order, reduce
-// the lanes of a row in double and round to f32 once: the oracle's exact
-// double sum up to ~2^-50 relative, so both agree bit for bit except in rare
-// rounding-boundary cases (<= 1 ulp). The single-weight and job-table forms
-// run the same kernel, so they agree bit for bit always.
+// sum over scale groups of scale * sum(code * x) exactly. x is written out as
+// base-256 integer digits, the digits' sums with the codes run on int8 matrix
+// instructions and are exact, integer sub-scales multiply them exactly, and a
+// double collects the blocks: the oracle's exact double sum up to ~2^-50
+// relative, so both agree bit for bit except in rare rounding-boundary cases
+// (<= 1 ulp). The order of a row's sums is fixed by its length alone, so the
+// single-weight and job-table forms agree bit for bit always. F32 and BF16
+// products are formed in double directly.
 //
-// Device layouts (split by the verified upload in uq_runtime.hip): a body
-// plane of 16-byte aligned units per row, a per-block fp16 scale plane, and an
-// aux plane (IQ4_XS block head, Q6_K scales in unit order); see frontier_layout.
+// Bound and choices (MI355X, HIP events over back-to-back launches, before ->
+// after, "before" being five v_dot4 digit planes with 8-16 lanes a row):
+//  * digits on the matrix core: v_dot4 needed 1.25 instructions and 5 bytes of
+//    LDS per weight; v_mfma_i32_16x16x64_i8 takes eight digits of 1,024 weights
+//    in one instruction and 0.25 bytes of LDS per weight. What is left on the
+//    VALU is the unpacking of the codes (IQ4/IQ3: 88 of 150 instructions a step
+//    of 16 rows x 256 columns), which bounds large IQ weights; Q6_K and Q8_0
+//    reach 5.4 and 4.7 TB/s of a 7.0 TB/s streaming read.
+//  * 52000 x 2560: Q6_K 38.8 -> 22.2 us, IQ3_XXS 32.8 -> 18.4, IQ4_NL 30.0 ->
+//    22.0, IQ4_XS 31.2 -> 18.4, Q8_0 30.8 -> 30.9. 256 x 16384: Q6_K 52.6 ->
+//    13.4, Q8_0 28.4 -> 17.6. 640 x 2560: IQ3_XXS 10.2 -> 4.8.
+//  * tiles of 16 rows are laid out at upload in the order in which a wave reads
+//    them (whole kilobytes per load instruction); Q8_0 shares the int8 matvec's
+//    row planes.
 #include "uq_device.h"
 #include "uq_internal.h"
 #include "../../include/uq.h"
@@ -132,34 +144,208 @@ __global__ __launch_bounds__(FWG) void k_dequant(const uint8_t* __restrict__ in,
 }
 
 // ---------------------------------------------------------------- layout repack / verify
-// Byte map of one GGUF block into the planes: map[o] = plane << 12 | offset
-// within that plane's block (plane 0 body, 1 aux, 2 fp16 scale).
-struct MapArgs {
-    uint16_t map[256];
-    int32_t block_bytes, plane_bytes[3];
+// 16-entry code books as v_perm_b32 tables. A selector byte q < 8 picks byte q
+// of the table; 8..11 give the sign of byte 1, 3, 5 or 7 (0x00 here, see below),
+// 12 gives 0x00 and 13..15 give 0xFF. With the codes 0..7 in one table and 8..15
+// in another, perm(first, q) ^ perm(second, q ^ 8) is the entry itself, or its
+// complement for (q & 7) >= 5: the tables hold those entries complemented. That
+// takes four instructions behind the masked nibbles where picking one of two
+// table bytes by bit 3 took five. The order of the codes makes bytes 1, 3, 5 and
+// 7 of both tables non-negative: values >= 0 at 1 and 3, values < 0
+// (complemented) at 5 and 7.
+struct Book {
+    uint32_t t[4];
+};
+constexpr int BOOK_ORDER[16] = {0, 8, 1, 9, 10, 2, 11, 3, 4, 12, 5, 13, 14, 6, 15, 7};  // code -> place in ascending order
+constexpr Book make_book(const int (&ascending)[16]) {
+    Book b{};
+    for (int q = 0; q < 16; q++) {
+        const int v = ascending[BOOK_ORDER[q]], e = (q & 7) >= 5 ? ~v : v;
+        b.t[q / 4] |= (uint32_t)(e & 255) << (8 * (q % 4));
+    }
+    return b;
+}
+constexpr int IQ4_VALUES[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
+constexpr int IQ3_VALUES[16] = {-62, -52, -44, -36, -28, -20, -12, -4, 4, 12, 20, 28, 36, 44, 52, 62};
+constexpr Book IQ4_BOOK = make_book(IQ4_VALUES), IQ3_BOOK = make_book(IQ3_VALUES);
+// place in ascending order -> code, four bits each
+constexpr uint64_t book_codes() {
+    uint64_t m = 0;
+    for (int q = 0; q < 16; q++) m |= (uint64_t)q << (4 * BOOK_ORDER[q]);
+    return m;
+}
+constexpr uint64_t book_places() {
+    uint64_t m = 0;
+    for (int q = 0; q < 16; q++) m |= (uint64_t)BOOK_ORDER[q] << (4 * q);
+    return m;
+}
+__device__ __forceinline__ uint32_t nibble_of(uint64_t table, uint32_t i) { return (uint32_t)(table >> (4 * i)) & 15u; }
+// both nibbles of a byte through a 16-entry table
+__device__ __forceinline__ uint32_t recode(uint64_t table, uint32_t b) {
+    return nibble_of(table, b & 15) | nibble_of(table, b >> 4) << 4;
+}
+
+struct LayoutArgs {
+    int64_t m;
+    int32_t kind, block_bytes, blocks;  // blocks per row
+    int32_t steps, bps;                 // steps per row, blocks per step
+    int32_t rec[3];                     // bytes of a tile's step in each plane
+    uint8_t* plane[3];
 };
 
-__global__ __launch_bounds__(FWG) void k_layout_repack(const uint8_t* __restrict__ src, int64_t blocks, MapArgs a,
-                                                       uint8_t* p0, uint8_t* p1, uint8_t* p2) {
-    const int64_t total = blocks * a.block_bytes;
-    for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < total; i += (int64_t)gridDim.x * FWG) {
-        const int64_t b = i / a.block_bytes;
-        const int o = (int)(i - b * a.block_bytes), e = a.map[o], pl = e >> 12, off = e & 0xfff;
-        uint8_t* dst = pl == 0 ? p0 : (pl == 1 ? p1 : p2);
-        dst[b * a.plane_bytes[pl] + off] = src[i];
+// Code of value e (0..31) of 32-value block sb of an IQ3_XXS superblock.
+__device__ __forceinline__ uint32_t iq3_code(const uint8_t* p, int sb, int e) {
+    const uint32_t s7 = (rd32(p + 66 + 4 * sb) >> (7 * (e / 8))) & 127u;
+    const uint32_t neg = ((s7 | (uint32_t)(__popc(s7) & 1) << 7) >> (e % 8)) & 1u;
+    const uint32_t level = ((c_iq3_grid[p[2 + 8 * sb + e / 4]] >> (8 * (e % 4))) & 255u) >> 3;
+    return nibble_of(book_codes(), neg ? 7 - level : 8 + level);
+}
+
+// Byte `at` of a tile's step in plane pl: what the block's bytes p (of the
+// lane's or row's own block) put there.
+__device__ uint32_t plane_byte(const LayoutArgs& a, const uint8_t* src, int pl, int64_t rec, int at) {
+    const int64_t tile = rec / a.steps;
+    const int t = (int)(rec - tile * a.steps);
+    const int sixth = a.rec[FL_ROW] == 160 && pl == FL_ROW;  // 16 x 8 scale bytes, then 16 x 2 bytes of d
+    int g = 0, r, o;  // lane group, row of the tile, byte of the record
+    if (pl == FL_BODY) {
+        const int lane = (at & 1023) >> 4;
+        g = lane >> 4;
+        r = lane & 15;
+        o = 16 * (at >> 10) + (at & 15);
+    } else if (pl == FL_LANE) {
+        const int w = a.rec[FL_LANE] / 64, lane = at / w;
+        g = lane >> 4;
+        r = lane & 15;
+        o = at - lane * w;
+    } else if (sixth && at < 128) {
+        r = at >> 3;
+        o = at & 7;
+    } else {
+        r = (sixth ? at - 128 : at) >> 1;
+        o = 8 + (at & 1);
+    }
+    const int64_t row = 16 * tile + r, b = (int64_t)t * a.bps + (a.bps > 1 ? g : 0);
+    if (row >= a.m || b >= a.blocks) return 0;
+    const uint8_t* p = src + (row * a.blocks + b) * a.block_bytes;
+    switch (a.kind) {
+    case KIND_IQ4_NL: return pl == FL_BODY ? recode(book_codes(), p[2 + o]) : p[o];
+    case KIND_IQ4_XS:
+        if (pl == FL_BODY) return recode(book_codes(), p[8 + 16 * (4 * (o >> 4) + g) + (o & 15)]);
+        if (o >= 8) return p[o - 8];
+        else {  // scale byte o: slice o >> 2, its block number o & 3
+            const int sb = 2 * (o & 3) + (o >> 2);
+            return (uint32_t)((int)((p[4 + sb / 2] >> (4 * (sb % 2))) & 15) + (int)(((rd16(p + 2) >> (2 * sb)) & 3) << 4) - 32) & 255u;
+        }
+    case KIND_IQ3_XXS:
+        if (pl == FL_BODY) {
+            const int sb = 4 * (o >> 4) + g;
+            return iq3_code(p, sb, o & 15) | iq3_code(p, sb, 16 + (o & 15)) << 4;
+        }
+        if (o >= 8) return p[o - 8];
+        return 2 * (p[66 + 4 * (2 * (o & 3) + (o >> 2)) + 3] >> 4) + 1;
+    default:  // Q6_K
+        if (pl == FL_BODY)
+            return o < 32 ? p[(g >> 1) * 64 + 32 * (o >> 4) + 16 * (g & 1) + (o & 15)]
+                          : p[128 + (g >> 1) * 32 + 16 * (g & 1) + (o & 15)];
+        return pl == FL_LANE ? p[192 + (g >> 1) * 8 + (g & 1) + 2 * o] : p[208 + o - 8];
     }
 }
 
-__global__ __launch_bounds__(FWG) void k_layout_verify(const uint8_t* __restrict__ src, int64_t blocks, MapArgs a,
-                                                       const uint8_t* p0, const uint8_t* p1, const uint8_t* p2,
+// One dword of a plane per thread; rows past the last and columns past n are zero.
+__global__ __launch_bounds__(FWG) void k_layout_repack(const uint8_t* __restrict__ src, LayoutArgs a, int pl, int64_t dwords) {
+    for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < dwords; i += (int64_t)gridDim.x * FWG) {
+        const int64_t rec = 4 * i / a.rec[pl];
+        const int at = (int)(4 * i - rec * a.rec[pl]);
+        uint32_t v = 0;
+#pragma unroll 1
+        for (int k = 0; k < 4; k++) v |= plane_byte(a, src, pl, rec, at + k) << (8 * k);
+        ((uint32_t*)a.plane[pl])[i] = v;
+    }
+}
+
+// Byte o of block b of a row as the planes hold it (-1: no GGUF bytes give them).
+__device__ int source_byte(const LayoutArgs& a, int64_t row, int64_t b, int o) {
+    const int64_t rec = (row >> 4) * a.steps + b / a.bps;
+    const int r = (int)(row & 15);
+    // the body byte `at` of lane group g's record
+    auto body = [&](int g, int at) {
+        return (uint32_t)a.plane[FL_BODY][rec * a.rec[FL_BODY] + 1024 * (at >> 4) + 16 * (16 * g + r) + (at & 15)];
+    };
+    auto scale = [&](int sb) { return (int)(int8_t)a.plane[FL_ROW][rec * 160 + 8 * r + 4 * (sb & 1) + (sb >> 1)]; };
+    switch (a.kind) {
+    case KIND_IQ4_NL: {
+        const int g = (int)(b % a.bps);
+        if (o < 2) return a.plane[FL_LANE][rec * 128 + 2 * (16 * g + r) + o];
+        return (int)recode(book_places(), body(g, o - 2));
+    }
+    case KIND_IQ4_XS:
+        if (o < 2) return a.plane[FL_ROW][rec * 160 + 128 + 2 * r + o];
+        if (o < 4) {  // scales_h: two high bits of blocks 4(o - 2) ..
+            int v = 0;
+            for (int k = 0; k < 4; k++) v |= (((scale(4 * (o - 2) + k) + 32) >> 4) & 3) << (2 * k);
+            return v;
+        }
+        if (o < 8) return ((scale(2 * (o - 4)) + 32) & 15) | ((scale(2 * (o - 4) + 1) + 32) & 15) << 4;
+        return (int)recode(book_places(), body(((o - 8) >> 4) & 3, 16 * ((o - 8) >> 6) + ((o - 8) & 15)));
+    case KIND_IQ3_XXS: {
+        if (o < 2) return a.plane[FL_ROW][rec * 160 + 128 + 2 * r + o];
+        // place in ascending order of value e of block sb: below 8 negative
+        auto place = [&](int sb, int e) {
+            return nibble_of(book_places(), (body(sb & 3, 16 * (sb >> 2) + (e & 15)) >> (4 * (e >> 4))) & 15u);
+        };
+        if (o < 66) {  // the grid index of four levels (the grid ascends)
+            const int sb = (o - 2) >> 3, e = 4 * ((o - 2) & 7);
+            uint32_t w = 0;
+            for (int k = 0; k < 4; k++) {
+                const uint32_t q = place(sb, e + k), level = q < 8 ? 7 - q : q - 8;
+                w |= (level == 7 ? 62u : 8 * level + 4) << (8 * k);
+            }
+            int lo = 0;
+            for (int step = 128; step; step >>= 1)
+                if (c_iq3_grid[lo + step] <= w) lo += step;
+            return c_iq3_grid[lo] == w ? lo : -1;
+        }
+        const int sb = (o - 66) >> 2;
+        uint32_t aux = (uint32_t)(scale(sb) >> 1) << 28;
+        bool even = (scale(sb) & 1) != 0;
+        for (int k = 0; k < 4; k++) {
+            uint32_t neg = 0;
+            for (int e = 0; e < 8; e++) neg |= (place(sb, 8 * k + e) < 8 ? 1u : 0u) << e;
+            even = even && (__popc(neg) & 1) == 0;
+            aux |= (neg & 127u) << (7 * k);
+        }
+        return even ? (int)((aux >> (8 * ((o - 66) & 3))) & 255u) : -1;
+    }
+    default: {  // Q6_K
+        if (o < 128) return (int)body(2 * (o >> 6) + ((o >> 4) & 1), 16 * ((o >> 5) & 1) + (o & 15));
+        if (o < 192) return (int)body(2 * ((o - 128) >> 5) + ((o >> 4) & 1), 32 + (o & 15));
+        if (o < 208) {
+            const int i = o - 192, g = 2 * (i >> 3) + (i & 1);
+            return a.plane[FL_LANE][rec * 256 + 4 * (16 * g + r) + ((i & 7) >> 1)];
+        }
+        return a.plane[FL_ROW][rec * 32 + 2 * r + (o - 208)];
+    }
+    }
+}
+
+__global__ __launch_bounds__(FWG) void k_layout_verify(const uint8_t* __restrict__ src, LayoutArgs a, int64_t total,
                                                        unsigned* bad) {
-    const int64_t total = blocks * a.block_bytes;
     unsigned miss = 0;
     for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < total; i += (int64_t)gridDim.x * FWG) {
-        const int64_t b = i / a.block_bytes;
-        const int o = (int)(i - b * a.block_bytes), e = a.map[o], pl = e >> 12, off = e & 0xfff;
-        const uint8_t* dst = pl == 0 ? p0 : (pl == 1 ? p1 : p2);
-        miss += dst[b * a.plane_bytes[pl] + off] != src[i];
+        const int64_t blk = i / a.block_bytes, row = blk / a.blocks;
+        miss += source_byte(a, row, blk - row * a.blocks, (int)(i - blk * a.block_bytes)) != (int)src[i];
+    }
+    if (miss) atomicAdd(bad, miss);
+}
+
+// F32 / BF16 rows against their copy
+__global__ __launch_bounds__(FWG) void k_copy_verify(const uint4* __restrict__ src, const uint4* __restrict__ dst,
+                                                     int64_t n, unsigned* bad) {
+    unsigned miss = 0;
+    for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < n; i += (int64_t)gridDim.x * FWG) {
+        const uint4 x = src[i], y = dst[i];
+        miss += (x.x != y.x) + (x.y != y.y) + (x.z != y.z) + (x.w != y.w);
     }
     if (miss) atomicAdd(bad, miss);
 }
@@ -168,181 +354,654 @@ __global__ __launch_bounds__(FWG) void k_layout_verify(const uint8_t* __restrict
 // Job of the launch (the FrontierJob of frontier_quant.cu:71-78 with the
 // planes of an uploaded weight): rows [0, m) of one weight times x.
 struct FJob {
-    const uint8_t* body;  // row r's units start at body + r * pitch
-    const uint8_t* aux;
-    const uint16_t* d;
+    const uint8_t* body;  // tiles (or, for F32, BF16 and Q8_0, rows of `pitch` bytes)
+    const uint8_t* lane;  // per-lane records of a tile's step
+    const uint8_t* row;   // per-row records of a tile's step (Q8_0: the fp16 scale plane)
     const float* x;
     float* y;
     int64_t m, pitch;
     int32_t kind, n;
-    int32_t wg0, wgs;  // first workgroup of the job, workgroups of the job
+    int32_t wg0, wgs;  // first workgroup of the job (JobArgs::start), workgroups of the job
 };
 
 // ---- exact integer form of x
-// Each 32-block of x is staged in LDS as integers X_j with x_j = X_j *
-// 2^(E - XSHIFT), E = max(biased exponent of max|x_j|, 1): X_j = m_j *
-// 2^(e_j - E + 14) for the 24-bit significand m_j, |X_j| < 2^38, exact when
-// every element lies within 2^14 of the block maximum (or its dropped low bits
-// are zero). X_j is held as five balanced base-256 digits in five byte planes,
-// so sum(code * X) over a block is five v_dot4 sums recombined exactly in
-// double (|sum| < 2^51). A block that is not exact (wider range, or a
-// non-finite value) is marked and its dots run in double from x itself.
-constexpr int XSHIFT = 164, NLIMB = 5;
+// x is staged in LDS as integers X_j with x_j = X_j * 2^(E - 188) in groups of
+// 256 values: E = max(biased exponent of max|x_j|, 1), |X_j| < 2^62, exact when
+// every element lies within 2^38 of the group's maximum (or has zeros in the
+// bits that fall away). X_j is held as eight balanced base-256 digits. A group that is
+// not exact (wider range, or a non-finite value) has digits 0 and a bit in
+// `wide`; its products run in double from x itself.
+//
+// The dots run on v_mfma_i32_16x16x64_i8 with the weights of 16 rows as one
+// operand and the digits as the other, so one instruction forms all eight
+// digits' sums of two scale groups for 16 rows, where v_dot4 needed eight
+// instructions a dword. The matrix core has 16 columns: eight digits of two
+// scale groups (slices). A column belongs to one slice, so the digits of the
+// other chunks in it are zeros.
+//
+// LDS: 16-value chunk c holds digit d as 16 bytes at XCHUNK*c + 16*d and 16 zero
+// bytes behind the eighth, which the column lanes of another slice read. The
+// stride of nine 16-byte slots spreads the staging's dword writes of one digit
+// over all banks (eight slots would put eight chunks on one bank).
+constexpr int XDIG = 8, XGROUP = 256, XCHUNK = 16 * (XDIG + 1);
 
 struct XStage {
-    const uint32_t* limb;  // NLIMB planes of n/16 16-byte chunks (16 elements), in unit-major slots
-    const int* bexp;       // per 32-block: E, or -1 when the block takes the double path
-    const float* xg;       // x in global memory (double path)
-    const float* xf;       // F32 / BF16 weights: x as f32 in LDS
-    int n4;                // n / 4: dwords per plane
+    const uint8_t* dig;
+    const double* gexp;   // per group: 2^(E - 188)
+    const float* xg;      // x in global memory (wide groups)
+    const float* xf;      // F32 / BF16 weights: x as f32 in LDS
+    uint64_t wide;        // bit g: group g runs in double
+    int n;
 };
 
-// Digit chunks are held unit-major: chunk k (elements 16k..16k+15) of the
-// job's kind sits in slot pos * NU + u, u its unit and pos its place in the
-// unit (NU units per row), so the lanes of a row group, which own
-// consecutive units, read consecutive 16-byte slots.
-__device__ __forceinline__ int chunk_slot(uint32_t kind, int k, int n) {
-    switch (kind) {
-    case KIND_Q6_K: {  // unit 4s + 2sub + h holds chunks 16s + 8sub + 2g + h, place g
-        const int u = 4 * (k >> 4) + 2 * ((k >> 3) & 1) + (k & 1);
-        return ((k >> 1) & 3) * (n / 64) + u;
-    }
-    case KIND_IQ3_XXS: return (k & 7) * (n / 128) + (k >> 3);
-    default: return (k & 1) * (n / 32) + (k >> 1);  // Q8_0, IQ4_NL, IQ4_XS: 2 chunks per unit
-    }
+// Four bytes of each of four dwords, byte k of all four in out[k].
+__device__ __forceinline__ void bytes_transposed(const uint32_t (&v)[4], uint32_t (&out)[4]) {
+    const uint32_t a01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400u);
+    const uint32_t a23 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400u);
+    const uint32_t b01 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602u);
+    const uint32_t b23 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
 }
 
-// sum(code * x) over NC chunks (4 dwords of packed signed codes each) in
-// slots slot0, slot0 + sstride, ...; e0 = first element (32-block exponent,
-// double path) and the chunks cover elements e0 + 16*c.
-template <int NC>
-__device__ __forceinline__ double seg_dot(const uint32_t (&c)[4 * NC], const XStage& xs, int e0, int slot0,
-                                          int sstride) {
-    const int E = xs.bexp[e0 >> 5];
-    if (E >= 0) {
-        int S[NLIMB];
+// The first groups of a wave, loaded ahead of its weights: loads return in
+// order, and x behind the weights would wait for HBM.
+constexpr int XAHEAD = 2;
+__device__ __forceinline__ float4 load_group(const float* __restrict__ x, int n, int grp) {
+    const int q = 64 * grp + ((int)threadIdx.x & 63);
+    return ((const float4*)x)[4 * q < n ? q : n / 4 - 1];
+}
+__device__ __forceinline__ void load_ahead(const float* __restrict__ x, int n, float4 (&v)[XAHEAD]) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
 #pragma unroll
-        for (int l = 0; l < NLIMB; l++) {
-            int a = 0;
+    for (int r = 0; r < XAHEAD; r++) v[r] = load_group(x, n, wave + r * nw);
+}
+
+// Stages x of one job, one 256-value group per wave at a time, 4 values per
+// lane; returns the wave's wide groups.
+__device__ __forceinline__ uint64_t stage_x(const float* __restrict__ x, int n, const float4 (&ahead)[XAHEAD], uint8_t* dig,
+                                            double* gexp) {
+    const int lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6, ng = (n + XGROUP - 1) / XGROUP;
+    uint64_t wide = 0;
+    const int first = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    auto group = [&](int grp, const float4& v4) {
+        const int q = 64 * grp + lane;
+        const float v[4] = {4 * q < n ? v4.x : 0.0f, 4 * q < n ? v4.y : 0.0f, 4 * q < n ? v4.z : 0.0f,
+                            4 * q < n ? v4.w : 0.0f};
+        const float amax = uq_group_max<64>(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        int E = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 255);
+        E = E < 1 ? 1 : (E > 254 ? 254 : E);
+        const double up = __builtin_bit_cast(double, (uint64_t)(188 - E + 1023) << 52);
+        bool ok = true;
+        uint32_t lo[4], hi[4];
 #pragma unroll
-            for (int ch = 0; ch < NC; ch++) {
-                const uint4 p = ((const uint4*)xs.limb)[l * (xs.n4 >> 2) + slot0 + ch * sstride];
-                a = uq_dot4((int)c[4 * ch + 0], (int)p.x, a);
-                a = uq_dot4((int)c[4 * ch + 1], (int)p.y, a);
-                a = uq_dot4((int)c[4 * ch + 2], (int)p.z, a);
-                a = uq_dot4((int)c[4 * ch + 3], (int)p.w, a);
-            }
-            S[l] = a;
+        for (int k = 0; k < 4; k++) {
+            // X = x * 2^(188 - E) as 2^32 * h + l, 0 <= l < 2^32: both exact, and X
+            // is whole where l has no fraction (not so for infinities and NaN)
+            const double X = (double)v[k] * up, h = __builtin_floor(X * 0x1p-32), l = __builtin_fma(h, -0x1p32, X);
+            ok = ok && l == __builtin_floor(l);
+            // offset binary: digit d = byte d of (X + 0x8080808080808080) - 0x80
+            const uint64_t Y = ((uint64_t)(uint32_t)(int)h << 32 | (uint32_t)l) + 0x8080808080808080ull;
+            lo[k] = (uint32_t)Y ^ 0x80808080u;
+            hi[k] = (uint32_t)(Y >> 32) ^ 0x80808080u;
         }
-        double t = (double)S[NLIMB - 1];
+        uint32_t d[8];
+        {
+            uint32_t t[4];
+            bytes_transposed(lo, t);
 #pragma unroll
-        for (int l = NLIMB - 2; l >= 0; l--) t = __builtin_fma(t, 256.0, (double)S[l]);
-        return __builtin_ldexp(t, E - XSHIFT);
-    }
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
+            for (int k = 0; k < 4; k++) d[k] = t[k];
+            bytes_transposed(hi, t);
 #pragma unroll
-    for (int q = 0; q < 4 * NC; q++)
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            s[k] = __builtin_fma((double)(int)(int8_t)(uint8_t)(c[q] >> (8 * k)), (double)xs.xg[e0 + 4 * q + k], s[k]);
-    return (s[0] + s[1]) + (s[2] + s[3]);
-}
-
-// Stages x of one job, 4 elements per thread (8 threads per 32-block): the
-// block's exponent from the 8-lane max of |x|, each X_j, and its five digits
-// packed 4 elements per dword into the five planes (byte l of X_j + 0x80 in
-// every digit position, minus 0x80: balanced digits in [-128, 127]).
-__device__ void stage_x(const float* __restrict__ x, int n, uint32_t kind, uint32_t* limb, int* bexp) {
-    const int n4 = n / 4;
-    for (int q = threadIdx.x; q < ((n4 + 7) & ~7); q += (int)blockDim.x) {
-        // q < n4 for the whole 8-lane group or for none of it (n % 32 == 0)
-        if (q < n4) {
-            const float4 v4 = ((const float4*)x)[q];
-            const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-            float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-            amax = uq_group_max<8>(amax);
-            int E = (int)(__builtin_bit_cast(uint32_t, amax) >> 23);
-            bool ok = E < 255 && !(amax != amax);
-            E = E < 1 ? 1 : E;
-            uint32_t lo[4], hi[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t bits = __builtin_bit_cast(uint32_t, v[k]);
-                const int eb = (int)((bits >> 23) & 255);
-                uint32_t m = bits & 0x7FFFFFu;
-                if (eb) m |= 0x800000u;
-                const int sh = (eb < 1 ? 1 : eb) - E + 14;
-                int64_t X = 0;
-                if (eb == 255) ok = false;
-                else if (sh >= 0) X = (int64_t)m << sh;
-                else if (sh > -24 && (m & ((1u << -sh) - 1u)) == 0) X = (int64_t)(m >> -sh);
-                else if (m != 0) ok = false;
-                if (bits >> 31) X = -X;
-                // offset binary: digit l = byte l of (X + 0x8080808080) - 0x80
-                const uint64_t Y = (uint64_t)(X + (int64_t)0x8080808080ll);
-                lo[k] = (uint32_t)Y ^ 0x80808080u;
-                hi[k] = (uint32_t)(Y >> 32) ^ 0x80u;
-            }
-            // 4x4 byte transpose of lo[] (plane l = byte l of each element), then plane 4
-            const uint32_t a01 = __builtin_amdgcn_perm(lo[1], lo[0], 0x05010400u);
-            const uint32_t a23 = __builtin_amdgcn_perm(lo[3], lo[2], 0x05010400u);
-            const uint32_t b01 = __builtin_amdgcn_perm(lo[1], lo[0], 0x07030602u);
-            const uint32_t b23 = __builtin_amdgcn_perm(lo[3], lo[2], 0x07030602u);
-            // a01 = [e0.b0, e1.b0, e0.b1, e1.b1], b01 = [e0.b2, e1.b2, e0.b3, e1.b3]
-            const int at = 4 * chunk_slot(kind, q >> 2, n) + (q & 3);  // dword within a plane
-            limb[0 * n4 + at] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
-            limb[1 * n4 + at] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
-            limb[2 * n4 + at] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
-            limb[3 * n4 + at] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
-            const uint32_t h01 = __builtin_amdgcn_perm(hi[1], hi[0], 0x0C0C0400u);
-            const uint32_t h23 = __builtin_amdgcn_perm(hi[3], hi[2], 0x0C0C0400u);
-            limb[4 * n4 + at] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
-            const bool all_ok = uq_group_max<8>(ok ? 0.0f : 1.0f) == 0.0f;
-            if ((q & 7) == 0) bexp[q >> 3] = all_ok ? E : -1;
+            for (int k = 0; k < 4; k++) d[4 + k] = t[k];
         }
-    }
+        if (__builtin_amdgcn_ballot_w64(!ok)) {
+            wide |= 1ull << grp;
+#pragma unroll
+            for (int k = 0; k < XDIG; k++) d[k] = 0;
+        }
+        const int c = q >> 2;
+#pragma unroll
+        for (int k = 0; k < XDIG; k++) *(uint32_t*)(dig + XCHUNK * c + 16 * k + 4 * (q & 3)) = d[k];
+        *(uint32_t*)(dig + XCHUNK * c + 16 * XDIG + 4 * (q & 3)) = 0;
+        if (lane == 0) gexp[grp] = __builtin_bit_cast(double, (uint64_t)(E - 188 + 1023) << 52);
+    };
+#pragma unroll
+    for (int r = 0; r < XAHEAD; r++)
+        if (first + r * nw < ng) group(first + r * nw, ahead[r]);
+#pragma unroll 1
+    for (int grp = first + XAHEAD * nw; grp < ng; grp += nw) group(grp, load_group(x, n, grp));
+    return wide;
 }
 
-// ---- per-kind unit readers
-// A lane owns units u = sub, sub + LPR, ... of a row; dot() returns the unit's
-// sum over scale groups of scale * sum(code * x).
+typedef int v4i __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4i as_v4i(const uint32_t (&c)[4]) { return v4i{(int)c[0], (int)c[1], (int)c[2], (int)c[3]}; }
+__device__ __forceinline__ v4i lds16(const uint8_t* p) { return *(const v4i*)p; }
 
-// 4 IQ4 codes of the low nibbles of the 4 bytes of `nib` (upper nibbles
-// ignored), packed as signed bytes: v_perm_b32 over each half of the code
-// book, then a third v_perm_b32 takes byte k from the half picked by bit 3 of
-// nibble k (selector k, or k + 4 for the upper half).
-__device__ __forceinline__ uint32_t iq4_lookup4(uint32_t nib, uint32_t t0, uint32_t t1, uint32_t t2, uint32_t t3) {
-    const uint32_t sel = nib & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(t1, t0, sel), hi = __builtin_amdgcn_perm(t3, t2, sel);
-    const uint32_t pick = ((nib >> 1) & 0x04040404u) | 0x03020100u;
-    return __builtin_amdgcn_perm(hi, lo, pick);
-}
-struct Iq4Book {
-    uint32_t t0, t1, t2, t3;
-    __device__ Iq4Book() {
-        const uint32_t* b = (const uint32_t*)c_iq4;
-        t0 = b[0];
-        t1 = b[1];
-        t2 = b[2];
-        t3 = b[3];
+// Lane roles. As an operand lane, lane l holds 16 codes of row l & 15 of the
+// tile, of the chunk that its lane group g = l >> 4 stands for, and 16 bytes of
+// column l & 15 = 8 * slice + digit of the digits. As a result lane it holds
+// four digits (4 * (g & 1) ..) of slice g >> 1 for row l & 15. Pair p of a set
+// of four chunks takes the chunks of lane groups 2p and 2p + 1 as its slices:
+// column lanes whose chunk is not their slice's read its zeros.
+struct Lane {
+    int lane, row, g;
+    int slot[2];  // byte offset in a chunk of the digit that this lane reads for pair p
+    __device__ __forceinline__ Lane() {
+        lane = (int)threadIdx.x & 63;
+        row = lane & 15;
+        g = lane >> 4;
+#pragma unroll
+        for (int p = 0; p < 2; p++) slot[p] = 16 * (g == 2 * p + (row >> 3) ? row & 7 : XDIG);
     }
 };
-// the 32 codes of one 16-byte IQ4 unit (low nibbles -> elements 0..15, high -> 16..31)
-__device__ __forceinline__ double iq4_dot32(const uint4& w, const XStage& xs, int u, const Iq4Book& bk) {
+// The value of lane groups (2p, 2p + 1) in the result lanes of slices (0, 1).
+__device__ __forceinline__ void to_slices(uint32_t v, uint32_t (&out)[2]) {
+    const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // [0 0 2 2], [1 1 3 3]
+    const auto b = __builtin_amdgcn_permlane32_swap(a[0], a[1], false, false);
+    out[0] = b[0];
+    out[1] = b[1];
+}
+
+// ---- per-kind steps
+// A wave walks a tile of 16 rows in steps of VPS columns; U is what a lane
+// loads for one step, NB how many steps are in flight. Two pay where the bytes
+// per instruction are many (Q8_0 and Q6_K, 52000 x 2560: 35.8 -> 30.9 us, 25.2 ->
+// 22.2); elsewhere, and for short waves (one_kernel), the smaller code of one
+// does (IQ4_XS 3001 x 2560: 5.10 -> 4.85 us; three or four are slower still). step() adds the step's products to the lane's four digit
+// sums; chunk() gives 16 codes, their first column and their scale for the
+// products of a wide group in double.
+
+// 16 codes of a 32-value block of nibbles through a code book: the low nibbles
+// are its values 0..15, the high ones 16..31.
+__device__ __forceinline__ void book_codes16(const Book& k, const uint4& w, int half, uint32_t (&c)[4]) {
     const uint32_t v[4] = {w.x, w.y, w.z, w.w};
-    uint32_t c[8];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        c[q] = iq4_lookup4(v[q], bk.t0, bk.t1, bk.t2, bk.t3);
-        c[4 + q] = iq4_lookup4(v[q] >> 4, bk.t0, bk.t1, bk.t2, bk.t3);
+        const uint32_t sel = (half ? v[q] >> 4 : v[q]) & 0x0F0F0F0Fu;
+        c[q] = __builtin_amdgcn_perm(k.t[1], k.t[0], sel) ^ __builtin_amdgcn_perm(k.t[3], k.t[2], sel ^ 0x08080808u);
     }
-    return seg_dot<2>(c, xs, 32 * u, u, xs.n4 / 8);
+}
+
+// A step runs in phases, kept apart by scheduling barriers: the digits of all
+// its products are read from LDS first, the codes are unpacked while those
+// reads are out, then the products go out back to back and their sums are
+// scaled. Left to itself the compiler reads each product's digits right before
+// it, and a wave spends its time waiting for LDS.
+__device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
+
+__device__ __forceinline__ v4i mfma64(const v4i& x, const v4i& w, const v4i& c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(x, w, c, 0, 0, 0);
+}
+
+// Four 32-value blocks (lane group g: block 4t + g) with an fp16 scale each.
+template <class T>
+__device__ __forceinline__ void step_f16(const typename T::U& u, const Lane& ln, const XStage& xs, int t, double (&acc)[4]) {
+    v4i x[2][2];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            x[p][h] = lds16(xs.dig + (2 * XCHUNK * ln.g + ln.slot[p]) + 8 * XCHUNK * t + h * XCHUNK);
+    const double e = xs.gexp[t >> 1];
+    phase();
+    uint32_t c0[4], c1[4], sc[2];
+    T::codes(u, 0, c0);
+    T::codes(u, 1, c1);
+    to_slices(__builtin_bit_cast(uint32_t, uq_half((uint16_t)u.d)), sc);
+    const v4i w0 = as_v4i(c0), w1 = as_v4i(c1), z = {0, 0, 0, 0};
+    v4i d[2];
+#pragma unroll
+    for (int p = 0; p < 2; p++) d[p] = mfma64(x[p][0], w0, z);
+#pragma unroll
+    for (int p = 0; p < 2; p++) d[p] = mfma64(x[p][1], w1, d[p]);
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const double s = (double)uq_bits_f(sc[p]) * e;
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i] = __builtin_fma((double)d[p][i], s, acc[i]);
+    }
+}
+
+// Eight 32-value blocks of a superblock (lane group g: blocks g and 4 + g):
+// products of the codes w with the digits x, each block's sums times its
+// integer scale.
+__device__ __forceinline__ void read_blocks(const Lane& ln, const XStage& xs, int t, v4i (&x)[2][2][2]) {
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                x[b][p][h] = lds16(xs.dig + (2 * XCHUNK * ln.g + ln.slot[p]) + 16 * XCHUNK * t + (8 * b + h) * XCHUNK);
+}
+__device__ __forceinline__ void block_sums(const v4i (&x)[2][2][2], const v4i (&w)[2][2], const int (&sc)[2][2], int (&ia)[4]) {
+    v4i d[2][2];
+    const v4i z = {0, 0, 0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) d[b][p] = mfma64(x[b][p][h], w[b][h], h ? d[b][p] : z);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        ia[i] = __mul24(sc[0][0], d[0][0][i]);
+        ia[i] += __mul24(sc[0][1], d[0][1][i]);
+        ia[i] += __mul24(sc[1][0], d[1][0][i]);
+        ia[i] += __mul24(sc[1][1], d[1][1][i]);
+    }
 }
 
 template <uint32_t K>
+struct TK;
+
+// Q8_0 shares the int8 matvec's row planes: a load instruction reads 64 bytes
+// (two blocks) of each of the tile's rows, lane group g their chunk g, so the
+// two halves of a block meet in one instruction and one column slice.
+template <>
+struct TK<KIND_Q8_0> {
+    static constexpr int VPS = 128, CHUNKS = 2, NB = 2;
+    struct U {
+        uint4 a, b;
+        uint32_t d;  // scale of block 4t + g
+    };
+    static __device__ __forceinline__ U load(const FJob& j, int64_t tile, int t, int lane) {
+        const int64_t r = 16 * tile + (lane & 15), rr = r < j.m - 1 ? r : j.m - 1;
+        const int c0 = VPS * t + 16 * (lane >> 4), c1 = c0 + 64, last = j.n - 16;
+        const int8_t* p = (const int8_t*)j.body + rr * j.pitch;
+        U u;
+        u.a = *(const uint4*)(p + (c0 < last ? c0 : last));
+        u.b = *(const uint4*)(p + (c1 < last ? c1 : last));
+        const int b = 4 * t + (lane >> 4), nb = j.n / 32;
+        const uint32_t d = ((const uint16_t*)j.row)[rr * nb + (b < nb ? b : nb - 1)];
+        u.d = b < nb ? d : 0u;
+        return u;
+    }
+    static __device__ __forceinline__ void step(const U& u, const Lane& ln, const XStage& xs, int t, double (&acc)[4]) {
+        const int slot = 16 * ((ln.g >> 1) == (ln.row >> 3) ? ln.row & 7 : XDIG);
+        v4i x[2];
+#pragma unroll
+        for (int p = 0; p < 2; p++) x[p] = lds16(xs.dig + (XCHUNK * ln.g + slot) + 8 * XCHUNK * t + 4 * XCHUNK * p);
+        const double e = xs.gexp[t >> 1];
+        phase();
+        uint32_t sc[2];
+        to_slices(__builtin_bit_cast(uint32_t, uq_half((uint16_t)u.d)), sc);
+        const uint32_t c0[4] = {u.a.x, u.a.y, u.a.z, u.a.w}, c1[4] = {u.b.x, u.b.y, u.b.z, u.b.w};
+        const v4i z = {0, 0, 0, 0};
+        const v4i d[2] = {mfma64(x[0], as_v4i(c0), z), mfma64(x[1], as_v4i(c1), z)};
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const double s = (double)uq_bits_f(sc[p]) * e;
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[i] = __builtin_fma((double)d[p][i], s, acc[i]);
+        }
+    }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
+        uint32_t sc[2];
+        to_slices(u.d, sc);
+        const uint4& w = k ? u.b : u.a;
+        c[0] = w.x, c[1] = w.y, c[2] = w.z, c[3] = w.w;
+        *col = VPS * t + 64 * k + 16 * ln.g;
+        return (double)uq_half((uint16_t)sc[k]);
+    }
+};
+
+template <>
+struct TK<KIND_IQ4_NL> {
+    static constexpr int VPS = 128, CHUNKS = 2, NB = 1;
+    struct U {
+        uint4 a;
+        uint32_t d;
+    };
+    static __device__ __forceinline__ U load(const FJob& j, int64_t tile, int t, int lane) {
+        const int64_t rec = tile * ((j.n + VPS - 1) / VPS) + t;
+        return {*(const uint4*)(j.body + rec * 1024 + (uint32_t)(16 * lane)),
+                *(const uint16_t*)(j.lane + rec * 128 + (uint32_t)(2 * lane))};
+    }
+    static __device__ __forceinline__ void codes(const U& u, int half, uint32_t (&c)[4]) { book_codes16(IQ4_BOOK, u.a, half, c); }
+    static __device__ __forceinline__ void step(const U& u, const Lane& ln, const XStage& xs, int t, double (&acc)[4]) {
+        step_f16<TK>(u, ln, xs, t, acc);
+    }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
+        codes(u, k, c);
+        *col = VPS * t + 32 * ln.g + 16 * k;
+        return (double)uq_half((uint16_t)u.d);
+    }
+};
+
+// The 256-value kinds: their sub-scales are small integers, so a step's digit
+// sums stay integers (|sum| < 2^27) and meet the double only once, with d.
+__device__ __forceinline__ void add_step(const int (&ia)[4], double s, double (&acc)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = __builtin_fma((double)ia[i], s, acc[i]);
+}
+
+// IQ4_XS, and IQ3_XXS with its grid and signs written out as codes of 4 bits (the
+// grid has eight levels): 35% more bytes than the grid indices, but those took
+// two dozen LDS lookups a step, and the lookups bounded the kernel (152000 x
+// 2560: 53 us against 43).
+template <uint32_t K>
+struct BookKind {
+    static constexpr int VPS = 256, CHUNKS = 4, NB = 1;
+    struct U {
+        uint4 a, b;  // blocks g and 4 + g of the superblock
+        uint32_t sc;  // scales of blocks s, 2 + s, 4 + s, 6 + s (s = g >> 1)
+        uint32_t d;
+    };
+    static constexpr Book book() { return K == KIND_IQ4_XS ? IQ4_BOOK : IQ3_BOOK; }
+    static constexpr float unit() { return K == KIND_IQ4_XS ? 1.0f : 0.25f; }  // IQ3: d (0.5 + s) / 2 = d/4 (2 s + 1)
+    static __device__ __forceinline__ U load(const FJob& j, int64_t tile, int t, int lane) {
+        const int64_t rec = tile * (j.n / VPS) + t;
+        const uint8_t* p = j.body + rec * 2048;
+        const uint32_t o = 16 * lane;
+        const uint8_t* r = j.row + rec * 160;
+        return {*(const uint4*)(p + o), *(const uint4*)(p + o + 1024),
+                *(const uint32_t*)(r + (uint32_t)(8 * (lane & 15) + 4 * (lane >> 5))),
+                *(const uint16_t*)(r + 128 + (uint32_t)(2 * (lane & 15)))};
+    }
+    static __device__ __forceinline__ double scale_d(const U& u) { return (double)(uq_half((uint16_t)u.d) * unit()); }
+    static __device__ __forceinline__ void step(const U& u, const Lane& ln, const XStage& xs, int t, double (&acc)[4]) {
+        v4i x[2][2][2];
+        read_blocks(ln, xs, t, x);
+        const double e = xs.gexp[t];
+        phase();
+        v4i w[2][2];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                uint32_t c[4];
+                book_codes16(book(), b ? u.b : u.a, h, c);
+                w[b][h] = as_v4i(c);
+            }
+        auto sc = [&](int k) { return (int)(int8_t)(uint8_t)(u.sc >> (8 * k)); };
+        const int si[2][2] = {{sc(0), sc(1)}, {sc(2), sc(3)}};
+        int ia[4];
+        block_sums(x, w, si, ia);
+        add_step(ia, scale_d(u) * e, acc);
+    }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
+        const int b = k >> 1;
+        book_codes16(book(), b ? u.b : u.a, 0, c);
+        if (k & 1) book_codes16(book(), b ? u.b : u.a, 1, c);
+        *col = VPS * t + 128 * b + 32 * ln.g + 16 * (k & 1);
+        // this lane's own block 4b + g: lane groups 2p, 2p + 1 stand for slices 0, 1 of pair p,
+        // and the scales of slice s sit in lane groups 2s and 2s + 1
+        const int own = 2 * b + (ln.g >> 1);
+        const uint32_t other = (uint32_t)__shfl((int)u.sc, ln.row + 32 * (ln.g & 1), 64);
+        return scale_d(u) * (double)(int8_t)(uint8_t)(other >> (8 * own));
+    }
+};
+template <>
+struct TK<KIND_IQ4_XS> : BookKind<KIND_IQ4_XS> {};
+template <>
+struct TK<KIND_IQ3_XXS> : BookKind<KIND_IQ3_XXS> {};
+
+// Q6_K unit g = 2*sub + h of a superblock: ql[sub*64 + 16h ..], ql[sub*64 + 32 + 16h ..],
+// qh[sub*32 + 16h ..] (16 bytes each) and the 4 group scales sc[sub*8 + h + 2k]: chunk k
+// holds columns 128*sub + 16h + 32k.
+template <>
+struct TK<KIND_Q6_K> {
+    static constexpr int VPS = 256, CHUNKS = 4, NB = 2;
+    struct U {
+        uint4 l0, l1, h;
+        uint32_t sc, d;
+    };
+    static __device__ __forceinline__ U load(const FJob& j, int64_t tile, int t, int lane) {
+        const int64_t rec = tile * (j.n / VPS) + t;
+        const uint8_t* p = j.body + rec * 3072;
+        const uint32_t o = 16 * lane;
+        return {*(const uint4*)(p + o), *(const uint4*)(p + o + 1024), *(const uint4*)(p + o + 2048),
+                *(const uint32_t*)(j.lane + rec * 256 + (uint32_t)(4 * lane)),
+                *(const uint16_t*)(j.row + rec * 32 + (uint32_t)(2 * (lane & 15)))};
+    }
+    static __device__ __forceinline__ void codes(const U& u, int k, uint32_t (&c)[4]) {
+        const uint4& l = (k & 1) ? u.l1 : u.l0;
+        const uint32_t lv[4] = {l.x, l.y, l.z, l.w}, hv[4] = {u.h.x, u.h.y, u.h.z, u.h.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t lo = (k < 2 ? lv[q] : lv[q] >> 4) & 0x0F0F0F0Fu;
+            const uint32_t hs = k < 2 ? hv[q] << (4 - 2 * k) : hv[q] >> (2 * k - 4);
+            // code - 32 as a signed byte: + 0x60 carries out of no byte, then flip bit 7
+            c[q] = (((hs & 0x30303030u) | lo) + 0x60606060u) ^ 0x80808080u;
+        }
+    }
+    static __device__ __forceinline__ void step(const U& u, const Lane& ln, const XStage& xs, int t, double (&acc)[4]) {
+        v4i x[4][2];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+                x[k][p] = lds16(xs.dig + (XCHUNK * (8 * (ln.g >> 1) + (ln.g & 1)) + ln.slot[p]) + 16 * XCHUNK * t + 2 * XCHUNK * k);
+        const double e = xs.gexp[t];
+        phase();
+        uint32_t sc[2];
+        to_slices(u.sc, sc);
+        const v4i z = {0, 0, 0, 0};
+        int ia[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 4; q += 2) {
+            v4i d[2][2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                uint32_t c[4];
+                codes(u, q + k, c);
+                const v4i w = as_v4i(c);
+#pragma unroll
+                for (int p = 0; p < 2; p++) d[k][p] = mfma64(x[q + k][p], w, z);
+            }
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    const int s = (int)(int8_t)(uint8_t)(sc[p] >> (8 * (q + k)));
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ia[i] += __mul24(s, d[k][p][i]);
+                }
+        }
+        add_step(ia, (double)uq_half((uint16_t)u.d) * e, acc);
+    }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
+        codes(u, 0, c);
+        if (k == 1) codes(u, 1, c);
+        if (k == 2) codes(u, 2, c);
+        if (k == 3) codes(u, 3, c);
+        *col = VPS * t + 128 * (ln.g >> 1) + 16 * (ln.g & 1) + 32 * k;
+        return (double)uq_half((uint16_t)u.d) * (double)(int8_t)(uint8_t)(u.sc >> (8 * k));
+    }
+};
+
+// Products of the groups in `mask` in double, steps [0, S) of the tile in
+// order: this lane's chunks of its row.
+template <class T>
+__device__ double wide_products(const FJob& j, int64_t tile, int S, uint64_t mask, const Lane& ln, const XStage& xs) {
+    double r = 0.0;
+#pragma unroll 1
+    for (int t = 0; t < S; t++) {
+        if (!((mask >> (t * T::VPS / XGROUP)) & 1)) continue;
+        const typename T::U u = T::load(j, tile, t, ln.lane);
+#pragma unroll 1
+        for (int k = 0; k < T::CHUNKS; k++) {
+            uint32_t c[4];
+            int col = 0;
+            const double s = T::chunk(u, ln, t, k, c, &col);
+            double d[4] = {0.0, 0.0, 0.0, 0.0};
+            if (col < xs.n) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const float4 x4 = *(const float4*)(xs.xg + col + 4 * q);
+                    const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        d[i] = __builtin_fma((double)(int)(int8_t)(uint8_t)(c[q] >> (8 * i)), (double)xv[i], d[i]);
+                }
+                r = __builtin_fma(s, (d[0] + d[1]) + (d[2] + d[3]), r);
+            }
+        }
+    }
+    return r;
+}
+
+// A tile's S steps fall into ns = min(8, S) column segments, which the eight
+// waves of a workgroup share out: with ns = 8 wave w takes segment (w + i) mod 8
+// of the workgroup's i-th tile, so that segments of unequal length even out,
+// with fewer every eighth segment of all its tiles. The segments' sums meet in
+// LDS, `dep` tiles at a time, and add up as a binary tree: a row's bits do not
+// depend on the launch, the number of its workgroups or the other jobs.
+constexpr int FL_SEGS = FL_WG / 64;
+
+// A wave's place: step s of segment seg (which ends at `end`) of tile i.
+struct Place {
+    int S, ns, inv;  // inv: x / ns = x * inv >> 8 for x < 16
+    int i, seg, s, end;
+    __device__ __forceinline__ void enter() {
+        s = ns == FL_SEGS ? seg * S >> 3 : seg;
+        end = ns == FL_SEGS ? (seg + 1) * S >> 3 : seg + 1;
+    }
+    __device__ __forceinline__ Place(int wave, int steps) {
+        S = steps;
+        ns = S < FL_SEGS ? S : FL_SEGS;
+        inv = 256 / ns + 1;
+        i = wave * inv >> 8;
+        seg = wave - i * ns;
+        enter();
+    }
+    __device__ __forceinline__ void next() {
+        if (ns == FL_SEGS) {
+            i++;
+            seg = (seg + 1) & (FL_SEGS - 1);
+        } else {
+            const int q = (seg + FL_SEGS) * inv >> 8;
+            i += q;
+            seg += FL_SEGS - q * ns;
+        }
+        enter();
+    }
+};
+
+// Tiles wgi, wgi + wgs, ... of one job. `stage` (the staging of x with its
+// barrier) runs once the wave's first loads are out. part: 2 x dep x FL_SEGS x
+// 64 doubles.
+template <class T, int NB, class F>
+__device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, double* part, F&& stage) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int S = (j.n + T::VPS - 1) / T::VPS, ns = S < FL_SEGS ? S : FL_SEGS;
+    const int tiles = (int)((j.m + 15) >> 4);
+    const int count = (tiles - wgi + j.wgs - 1) / j.wgs;  // this workgroup's tiles
+    const Lane ln;
+    const double half = (ln.g & 1) ? 4294967296.0 : 1.0;  // digits 4..7 stand 2^32 higher
+    // A fetch past the wave's last step reads one address in every lane instead
+    // of being branched around: with the same loads on every path the
+    // compiler's waits stay exact (a branch made them wait for every load).
+    typename T::U buf[NB];
+    Place f(wave, S);
+    auto fetch = [&](typename T::U& b) {
+        const bool on = f.i < count;
+        b = T::load(j, on ? wgi + f.i * j.wgs : 0, on ? f.s : 0, on ? ln.lane : 0);
+        if (++f.s >= f.end) f.next();
+    };
+#pragma unroll
+    for (int b = 0; b < NB; b++) fetch(buf[b]);
+    const XStage xs = stage();
+    // Tiles [from, to) of the workgroup: one wave sums a tile's segments, then
+    // its four lane groups.
+    bool nan = false;
+    auto sum_tiles = [&](int from, int to, int buffer, uint64_t mask) {
+        __syncthreads();
+        for (int i = from + wave; i < to; i += FL_SEGS) {
+            double v[FL_SEGS];
+#pragma unroll
+            for (int k = 0; k < FL_SEGS; k++) {
+                const double t = part[((buffer * dep + (i - from)) * FL_SEGS + k) * 64 + ln.lane];
+                v[k] = k < ns ? t : 0.0;
+            }
+            double top = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
+            if (mask) top += wide_products<T>(j, tile, S, mask, ln, xs);
+            const double sum = uq_swap32_sum(uq_swap16_sum(top));
+            nan = nan || sum != sum;
+            if (ln.g == 0 && row < j.m) j.y[row] = (float)sum;
+        }
+    };
+    auto combine = [&](const double (&acc)[4]) {
+        double t = __builtin_fma(acc[3], 256.0, acc[2]);
+        t = __builtin_fma(t, 256.0, acc[1]);
+        return __builtin_fma(t, 256.0, acc[0]) * half;
+    };
+    Place p(wave, S);
+    if (xs.wide == 0) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+        int base = 0, buffer = 0;
+        // once the wave is past them, the workgroup sums the tiles from `base` on
+        auto flush = [&]() {
+            const int to = base + dep < count ? base + dep : count;
+            sum_tiles(base, to, buffer, 0);
+            base = to;
+            buffer ^= 1;
+        };
+        auto catch_up = [&]() {
+#pragma unroll 1
+            while (p.i >= base + dep && p.i < count) flush();
+        };
+        catch_up();
+        while (p.i < count) {
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                // (a step past the last is skipped, its fetch is not: a loop left
+                // from the middle would cost the waits their counts as well)
+                const bool on = p.i < count;
+                if (on) T::step(buf[b], ln, xs, p.s, acc);
+                fetch(buf[b]);
+                if (on && ++p.s == p.end) {
+                    part[((buffer * dep + (p.i - base)) * FL_SEGS + p.seg) * 64 + ln.lane] = combine(acc);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[i] = 0.0;
+                    p.next();
+                    catch_up();
+                }
+            }
+        }
+#pragma unroll 1
+        while (base < count) flush();
+        // A zero digit times an infinite scale is NaN where the row's own
+        // products are not: the tiles of a wave that saw one run again, wholly
+        // in double.
+        if (__builtin_amdgcn_ballot_w64(nan) == 0) return;
+#pragma unroll 1
+        for (int i = 0; i < count; i++) {
+            if (((i % dep) & (FL_SEGS - 1)) != wave) continue;
+            const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
+            const double sum = uq_swap32_sum(uq_swap16_sum(wide_products<T>(j, tile, S, ~0ull, ln, xs)));
+            if (ln.g == 0 && row < j.m) j.y[row] = (float)sum;
+        }
+        return;
+    }
+    // Some group of x is wide: without the ring, tile by tile.
+#pragma unroll 1
+    for (int i = 0; i < count; i++) {
+        if (p.i == i) {
+            double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+            for (; p.s < p.end; p.s++) {
+                const typename T::U u = T::load(j, wgi + i * j.wgs, p.s, ln.lane);
+                T::step(u, ln, xs, p.s, acc);
+            }
+            part[((i & 1) * dep * FL_SEGS + p.seg) * 64 + ln.lane] = combine(acc);
+            p.next();
+        }
+        sum_tiles(i, i + 1, i & 1, xs.wide);
+    }
+}
+
+// ---- F32 / BF16 rows
+// A lane owns units u = sub, sub + LPR, ... of a row; dot() returns the unit's
+// products with x in double.
+template <uint32_t K>
 struct FK;
 
-// F32 / BF16 weights are not small-integer codes: products in double from x.
 template <>
 struct FK<KIND_F32> {
     static constexpr int WPU = 8, LPR = 64, CH = 4;
@@ -353,7 +1012,7 @@ struct FK<KIND_F32> {
         const uint4* p = (const uint4*)(j.body + row * j.pitch) + 2 * u;
         return {p[0], p[1]};
     }
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t*, const Iq4Book&) {
+    static __device__ double dot(const U& v, const XStage& xs, int u) {
         const float* x = xs.xf + 8 * u;
         const float4 xa = ((const float4*)x)[0], xb = ((const float4*)x)[1];
         const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
@@ -374,7 +1033,7 @@ struct FK<KIND_BF16> {
     static __device__ U load(const FJob& j, int64_t row, int u) {
         return {((const uint4*)(j.body + row * j.pitch))[u]};
     }
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t*, const Iq4Book&) {
+    static __device__ double dot(const U& v, const XStage& xs, int u) {
         const float* x = xs.xf + 8 * u;
         const float4 xa = ((const float4*)x)[0], xb = ((const float4*)x)[1];
         const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
@@ -389,133 +1048,6 @@ struct FK<KIND_BF16> {
     }
 };
 
-template <>
-struct FK<KIND_Q8_0> {
-    static constexpr int WPU = 32, LPR = 16, CH = 4;
-    struct U {
-        uint4 a, b;
-        uint32_t d;
-    };
-    static __device__ U load(const FJob& j, int64_t row, int u) {
-        const uint4* p = (const uint4*)(j.body + row * j.pitch) + 2 * u;
-        return {p[0], p[1], j.d[row * (j.n / 32) + u]};
-    }
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t*, const Iq4Book&) {
-        const uint32_t c[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
-        return (double)uq_half((uint16_t)v.d) * seg_dot<2>(c, xs, 32 * u, u, xs.n4 / 8);
-    }
-};
-
-template <>
-struct FK<KIND_IQ4_NL> {
-    static constexpr int WPU = 32, LPR = 16, CH = 4;
-    struct U {
-        uint4 a;
-        uint32_t d;
-    };
-    static __device__ U load(const FJob& j, int64_t row, int u) {
-        return {((const uint4*)(j.body + row * j.pitch))[u], j.d[row * (j.n / 32) + u]};
-    }
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t*, const Iq4Book& bk) {
-        return (double)uq_half((uint16_t)v.d) * iq4_dot32(v.a, xs, u, bk);
-    }
-};
-
-template <>
-struct FK<KIND_IQ4_XS> {
-    static constexpr int WPU = 32, LPR = 16, CH = 4;
-    struct U {
-        uint4 a;
-        uint2 h;  // block head: d | scales_h << 16, scales_l
-    };
-    static __device__ U load(const FJob& j, int64_t row, int u) {
-        const uint2 h = ((const uint2*)j.aux)[row * (j.n / 256) + u / 8];
-        return {((const uint4*)(j.body + row * j.pitch))[u], h};
-    }
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t*, const Iq4Book& bk) {
-        const int sb = u & 7;
-        const int sc = (int)((v.h.y >> (4 * sb)) & 15) | (int)(((v.h.x >> (16 + 2 * sb)) & 3) << 4);
-        const float scale = uq_half((uint16_t)(v.h.x & 0xFFFF)) * (float)(sc - 32);
-        return (double)scale * iq4_dot32(v.a, xs, u, bk);
-    }
-};
-
-// Q6_K unit k = 2*sub + h of a superblock: ql[sub*64 + 16h ..], ql[sub*64 + 32 + 16h ..],
-// qh[sub*32 + 16h ..] (16 bytes each) and the 4 group scales sc[sub*8 + h + 2g].
-template <>
-struct FK<KIND_Q6_K> {
-    static constexpr int WPU = 64, LPR = 8, CH = 2;
-    struct U {
-        uint4 l0, l1, h;
-        uint32_t sc, d;
-    };
-    static __device__ U load(const FJob& j, int64_t row, int u) {
-        const uint4* p = (const uint4*)(j.body + row * j.pitch) + 3 * u;
-        const uint32_t sc = ((const uint32_t*)j.aux)[row * (j.n / 64) + u];
-        return {p[0], p[1], p[2], sc, j.d[row * (j.n / 256) + u / 4]};
-    }
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t*, const Iq4Book&) {
-        const int e0 = 256 * (u >> 2) + 128 * ((u >> 1) & 1) + 16 * (u & 1);
-        const float d = uq_half((uint16_t)v.d);
-        const uint32_t l0[4] = {v.l0.x, v.l0.y, v.l0.z, v.l0.w}, l1[4] = {v.l1.x, v.l1.y, v.l1.z, v.l1.w};
-        const uint32_t hh[4] = {v.h.x, v.h.y, v.h.z, v.h.w};
-        double r = 0.0;
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            uint32_t c[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint32_t lo = ((g & 1 ? l1[q] : l0[q]) >> (4 * (g >> 1))) & 0x0F0F0F0Fu;
-                // 6-bit code with bit 5 flipped, its sign bit copied to bits 6-7: code - 32
-                const uint32_t t = (lo | (((hh[q] >> (2 * g)) & 0x03030303u) << 4)) ^ 0x20202020u;
-                const uint32_t s5 = t & 0x20202020u;
-                c[q] = t | (s5 << 1) | (s5 << 2);
-            }
-            const float scale = d * (float)(int8_t)(uint8_t)(v.sc >> (8 * g));
-            r = __builtin_fma((double)scale, seg_dot<1>(c, xs, e0 + 32 * g, g * (xs.n4 / 16) + u, 0), r);
-        }
-        return r;
-    }
-};
-
-// IQ3_XXS unit k of a superblock: grid indices of sub-blocks 4k..4k+3 (32
-// bytes) then their 4 sign/scale words (16 bytes).
-template <>
-struct FK<KIND_IQ3_XXS> {
-    static constexpr int WPU = 128, LPR = 8, CH = 2;
-    struct U {
-        uint4 q0, q1, a;
-        uint32_t d;
-    };
-    static __device__ U load(const FJob& j, int64_t row, int u) {
-        const uint4* p = (const uint4*)(j.body + row * j.pitch) + 3 * u;
-        return {p[0], p[1], p[2], j.d[row * (j.n / 256) + u / 2]};
-    }
-    // grid bytes (<= 62) negated where the sign mask byte is 0xFF: (g ^ m) + (m & 1),
-    // with no carry between bytes
-    static __device__ double dot(const U& v, const XStage& xs, int u, const uint32_t* grid, const Iq4Book&) {
-        const float d = uq_half((uint16_t)v.d);
-        const uint32_t qs[8] = {v.q0.x, v.q0.y, v.q0.z, v.q0.w, v.q1.x, v.q1.y, v.q1.z, v.q1.w};
-        const uint32_t aux[4] = {v.a.x, v.a.y, v.a.z, v.a.w};
-        double r = 0.0;
-#pragma unroll
-        for (int l = 0; l < 4; l++) {
-            uint32_t c[8];
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const uint4 sm = ((const uint4*)(grid + 256))[(aux[l] >> (7 * g)) & 127u];
-                const uint32_t word = qs[2 * l + (g >> 1)];
-                const uint32_t g0 = grid[(word >> (16 * (g & 1))) & 255], g1 = grid[(word >> (16 * (g & 1) + 8)) & 255];
-                c[2 * g] = (g0 ^ sm.x) + sm.z;
-                c[2 * g + 1] = (g1 ^ sm.y) + sm.w;
-            }
-            const float scale = d * (0.5f + (float)(aux[l] >> 28)) * 0.5f;
-            r = __builtin_fma((double)scale, seg_dot<2>(c, xs, 128 * u + 32 * l, 2 * l * (xs.n4 / 32) + u, xs.n4 / 32), r);
-        }
-        return r;
-    }
-};
-
 // Rows of one job for workgroup `wgi` of `wgc`: LPR lanes per row, 64/LPR
 // rows per wave, row blocks wgi, wgi + wgc, ... A lane owns units u = sub +
 // LPR*i of its row and walks them in chunks of CH units: the next chunk's
@@ -523,7 +1055,7 @@ struct FK<KIND_IQ3_XXS> {
 // current chunk's dots. Per row the lane adds its units in order; the lane
 // group sums in double and rounds once.
 template <class T>
-__device__ void job_rows(const FJob& j, int wgi, int wgc, const XStage& xs, const uint32_t* grid) {
+__device__ void job_rows(const FJob& j, int wgi, int wgc, const XStage& xs) {
     constexpr int LPR = T::LPR, CH = T::CH, RPW = 64 / LPR;
     const int RPB = RPW * (int)(blockDim.x / 64);  // rows per row block: the launch picks 256 or 512 threads
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane % LPR, grp = lane / LPR;
@@ -532,7 +1064,6 @@ __device__ void job_rows(const FJob& j, int wgi, int wgc, const XStage& xs, cons
     const int nch = (nb + CH - 1) / CH;      // chunks per row
     const int64_t rblocks = (j.m + RPB - 1) / RPB;
     if (wgi >= rblocks) return;
-    const Iq4Book bk;
     typename T::U buf[2][CH];
     // (row block, chunk) of the next fetch, advanced without division
     int64_t frb = wgi;
@@ -564,7 +1095,7 @@ __device__ void job_rows(const FJob& j, int wgi, int wgc, const XStage& xs, cons
                 for (int k = 0; k < CH; k++) {
                     const int u = sub + LPR * (c * CH + k);
                     if (c * CH + k < nb) {
-                        const double d = T::dot(buf[h][k], xs, u < nu ? u : nu - 1, grid, bk);
+                        const double d = T::dot(buf[h][k], xs, u < nu ? u : nu - 1);
                         acc = acc + (u < nu ? d : 0.0);
                     }
                 }
@@ -590,107 +1121,134 @@ constexpr int rows_per_wave() {
 // (no device table to copy before the launch); longer tables take several
 // launches, each row computed the same way.
 constexpr int MAX_JOBS = 32;
+struct Parts {
+    int32_t dep, at;  // tiles whose segments meet at once; their place in LDS
+};
 struct JobArgs {
+    Parts parts;
+    int32_t start[MAX_JOBS];  // first workgroup of each job, ascending; past the last job INT32_MAX
     FJob job[MAX_JOBS];
-    int count;
 };
 
-// Shared front of the linear kernels: the workgroup's job (wg0 ascending)
-// and its staged x.
-__device__ __forceinline__ FJob find_job(const JobArgs& a) {
-    int lo = 0, hi = a.count;
-    while (lo + 1 < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (a.job[mid].wg0 <= (int)blockIdx.x) lo = mid;
-        else hi = mid;
+// The workgroup's job and its place in it (-1: none). The arguments lie in host
+// memory and the first read of each line takes about a microsecond, so the
+// workgroup reads as few as it can one behind the other: with a grid row per job
+// the job's record alone, otherwise all starts at once (a binary search over the
+// jobs was five such reads).
+__device__ __forceinline__ FJob find_job(const JobArgs& a, int* wgi) {
+    int job = (int)blockIdx.y;
+    if (gridDim.y == 1) {
+        const int32_t s = a.start[threadIdx.x & (MAX_JOBS - 1)];
+        job = __popc((uint32_t)__builtin_amdgcn_ballot_w64(s <= (int32_t)blockIdx.x)) - 1;
     }
-    return a.job[lo];
+    const FJob j = a.job[job];
+    *wgi = gridDim.y == 1 ? (int)blockIdx.x - j.wg0 : ((int)blockIdx.x < j.wgs ? (int)blockIdx.x : -1);
+    return j;
 }
-template <bool INTS>
-__device__ __forceinline__ XStage stage_job(const FJob& j, uint32_t* fl_lds, uint32_t* lgrid) {
-    XStage xs;
-    xs.limb = fl_lds;
-    xs.bexp = (const int*)(fl_lds + NLIMB * (j.n / 4));
-    xs.xg = j.x;
-    xs.xf = (const float*)fl_lds;
-    xs.n4 = j.n / 4;
-    if (INTS) stage_x(j.x, j.n, (uint32_t)j.kind, fl_lds, (int*)(fl_lds + NLIMB * (j.n / 4)));
-    else
-        for (int i = threadIdx.x; i < j.n / 4; i += (int)blockDim.x) ((float4*)fl_lds)[i] = ((const float4*)j.x)[i];
-    for (int i = threadIdx.x; i < 256; i += (int)blockDim.x) lgrid[i] = c_iq3_grid[i];
-    // IQ3_XXS signs after the grid: entry s7 (7 stored sign bits, the 8th their
-    // parity) = byte masks of values 0-3 and 4-7 (0xFF = negative) and the
-    // masks' low bits
-    for (int i = threadIdx.x; i < 128; i += (int)blockDim.x) {
-        const uint32_t sg = (uint32_t)i | ((uint32_t)(__popc(i) & 1) << 7);
-        uint32_t m[2];
-        for (int h = 0; h < 2; h++) {
-            uint32_t v = 0;
-            for (int k = 0; k < 4; k++)
-                if ((sg >> (4 * h + k)) & 1) v |= 0xFFu << (8 * k);
-            m[h] = v;
-        }
-        ((uint4*)(lgrid + 256))[i] = make_uint4(m[0], m[1], m[0] & 0x01010101u, m[1] & 0x01010101u);
-    }
+// Dynamic LDS of a job: the digits of x padded to whole groups and the group
+// factors (F32 / BF16 weights: x as f32).
+__device__ __forceinline__ XStage stage_floats(const FJob& j, uint8_t* lds) {
+    XStage xs{};
+    xs.xf = (const float*)lds;
+    xs.n = j.n;
+    for (int i = threadIdx.x; i < j.n / 4; i += (int)blockDim.x) ((float4*)lds)[i] = ((const float4*)j.x)[i];
     __syncthreads();
     return xs;
 }
-
-// Jobs of one kind: registers sized for that kind alone.
-template <uint32_t K>
-__global__ __launch_bounds__(FL_WG) void k_flinear_kind(JobArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint32_t fl_lds[];
-    __shared__ __attribute__((aligned(16))) uint32_t lgrid[256 + 4 * 128];  // IQ3 grid, then the sign table
-    const FJob j = find_job(a);
-    const XStage xs = stage_job<K != KIND_F32 && K != KIND_BF16>(j, fl_lds, lgrid);
-    job_rows<FK<K>>(j, (int)blockIdx.x - j.wg0, j.wgs, xs, lgrid);
+__device__ __forceinline__ XStage stage_digits(const FJob& j, const float4 (&ahead)[XAHEAD], uint8_t* lds, uint64_t* wides) {
+    const int ng = (j.n + XGROUP - 1) / XGROUP;
+    uint8_t* const dig = lds;
+    double* const gexp = (double*)(lds + XCHUNK * (XGROUP / 16) * ng);
+    const uint64_t wide = stage_x(j.x, j.n, ahead, dig, gexp);
+    if ((threadIdx.x & 63) == 0) wides[threadIdx.x >> 6] = wide;
+    __syncthreads();
+    XStage xs{};
+    xs.dig = dig;
+    xs.gexp = gexp;
+    xs.xg = j.x;
+    xs.n = j.n;
+    uint64_t all = 0;
+    for (int w = 0; w < (int)blockDim.x / 64; w++) all |= wides[w];
+    // the same in every lane: a scalar mask
+    xs.wide = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)all) |
+              (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(all >> 32)) << 32;
+    return xs;
+}
+template <uint32_t K, int NB = 0>
+__device__ __forceinline__ void run_job(const FJob& j, int wgi, const Parts& parts, uint8_t* lds, uint64_t* wides) {
+    if constexpr (K == KIND_F32 || K == KIND_BF16) {
+        const XStage xs = stage_floats(j, lds);
+        job_rows<FK<K>>(j, wgi, j.wgs, xs);
+    } else {
+        float4 ahead[XAHEAD];
+        load_ahead(j.x, j.n, ahead);
+        job_tiles<TK<K>, NB ? NB : TK<K>::NB>(j, wgi, parts.dep, (double*)(lds + parts.at), [&]() { return stage_digits(j, ahead, lds, wides); });
+    }
 }
 
-// One launch over a job table of mixed kinds (wg0 ascending): the workgroup finds its job,
-// stages that job's x (integer digit planes and block exponents) and the IQ3
-// grid in LDS, and runs its rows. Dynamic LDS: NLIMB * n + 4 * (n / 32) bytes
-// (F32 / BF16 weights: x as 4 * n bytes of f32).
-__global__ __launch_bounds__(FL_WG) void k_flinear(JobArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint32_t fl_lds[];
-    __shared__ __attribute__((aligned(16))) uint32_t lgrid[256 + 4 * 128];  // IQ3 grid, then the sign table
-    const FJob j = find_job(a);
-    const int wgi = (int)blockIdx.x - j.wg0, wgc = j.wgs;
-    if (j.kind == KIND_F32 || j.kind == KIND_BF16) {
-        const XStage xs = stage_job<false>(j, fl_lds, lgrid);
-        if (j.kind == KIND_F32) job_rows<FK<KIND_F32>>(j, wgi, wgc, xs, lgrid);
-        else job_rows<FK<KIND_BF16>>(j, wgi, wgc, xs, lgrid);
-        return;
-    }
-    const XStage xs = stage_job<true>(j, fl_lds, lgrid);
+// One job, its record in the first lines of the arguments (four waves per SIMD:
+// two workgroups of a CU at work; the row kinds hold more).
+struct OneJob {
+    Parts parts;
+    FJob job;
+};
+template <uint32_t K, int NB = 0>
+__global__ __launch_bounds__(FL_WG, 4) void k_flinear_one(OneJob a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t fl_lds[];
+    __shared__ uint64_t wides[FL_SEGS];
+    run_job<K, NB>(a.job, (int)blockIdx.x, a.parts, fl_lds, wides);
+}
+
+// A job table of F32 or BF16 weights: registers sized for that kind alone.
+template <uint32_t K>
+__global__ __launch_bounds__(FL_WG, 4) void k_flinear_rows(JobArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t fl_lds[];
+    int wgi;
+    const FJob j = find_job(a, &wgi);
+    if (wgi >= 0) run_job<K>(j, wgi, a.parts, fl_lds, nullptr);
+}
+
+// One launch over a job table of any kinds.
+__global__ __launch_bounds__(FL_WG, 4) void k_flinear(JobArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t fl_lds[];
+    __shared__ uint64_t wides[FL_SEGS];
+    int wgi;
+    const FJob j = find_job(a, &wgi);
+    if (wgi < 0) return;
     switch (j.kind) {
-    case KIND_Q8_0: job_rows<FK<KIND_Q8_0>>(j, wgi, wgc, xs, lgrid); break;
-    case KIND_IQ4_NL: job_rows<FK<KIND_IQ4_NL>>(j, wgi, wgc, xs, lgrid); break;
-    case KIND_IQ4_XS: job_rows<FK<KIND_IQ4_XS>>(j, wgi, wgc, xs, lgrid); break;
-    case KIND_Q6_K: job_rows<FK<KIND_Q6_K>>(j, wgi, wgc, xs, lgrid); break;
-    case KIND_IQ3_XXS: job_rows<FK<KIND_IQ3_XXS>>(j, wgi, wgc, xs, lgrid); break;
+    case KIND_F32: run_job<KIND_F32>(j, wgi, a.parts, fl_lds, wides); break;
+    case KIND_BF16: run_job<KIND_BF16>(j, wgi, a.parts, fl_lds, wides); break;
+    case KIND_Q8_0: run_job<KIND_Q8_0>(j, wgi, a.parts, fl_lds, wides); break;
+    case KIND_IQ4_NL: run_job<KIND_IQ4_NL>(j, wgi, a.parts, fl_lds, wides); break;
+    case KIND_IQ4_XS: run_job<KIND_IQ4_XS>(j, wgi, a.parts, fl_lds, wides); break;
+    case KIND_Q6_K: run_job<KIND_Q6_K>(j, wgi, a.parts, fl_lds, wides); break;
+    case KIND_IQ3_XXS: run_job<KIND_IQ3_XXS>(j, wgi, a.parts, fl_lds, wides); break;
     default: break;
     }
 }
 
-// The kernel for a job table: the kind's own kernel when every job has that kind.
-using FlKernel = void (*)(JobArgs);
-FlKernel kernel_for(const JobArgs& a) {
-    const int32_t k = a.job[0].kind;
-    for (int i = 1; i < a.count; i++)
-        if (a.job[i].kind != k) return k_flinear;
-    switch (k) {
-    case KIND_F32: return k_flinear_kind<KIND_F32>;
-    case KIND_BF16: return k_flinear_kind<KIND_BF16>;
-    case KIND_Q8_0: return k_flinear_kind<KIND_Q8_0>;
-    case KIND_IQ4_NL: return k_flinear_kind<KIND_IQ4_NL>;
-    case KIND_IQ4_XS: return k_flinear_kind<KIND_IQ4_XS>;
-    case KIND_Q6_K: return k_flinear_kind<KIND_Q6_K>;
-    case KIND_IQ3_XXS: return k_flinear_kind<KIND_IQ3_XXS>;
+using OneKernel = void (*)(OneJob);
+using TableKernel = void (*)(JobArgs);
+// `few`: no wave has more than two steps.
+OneKernel one_kernel(int32_t kind, bool few) {
+    switch (kind) {
+    case KIND_F32: return k_flinear_one<KIND_F32>;
+    case KIND_BF16: return k_flinear_one<KIND_BF16>;
+    case KIND_Q8_0: return few ? k_flinear_one<KIND_Q8_0, 1> : k_flinear_one<KIND_Q8_0>;
+    case KIND_IQ4_NL: return k_flinear_one<KIND_IQ4_NL>;
+    case KIND_IQ4_XS: return k_flinear_one<KIND_IQ4_XS>;
+    case KIND_Q6_K: return few ? k_flinear_one<KIND_Q6_K, 1> : k_flinear_one<KIND_Q6_K>;
     }
-    return k_flinear;
+    return k_flinear_one<KIND_IQ3_XXS>;
+}
+TableKernel table_kernel(const JobArgs& a, int count) {
+    const int32_t k = a.job[0].kind;
+    for (int i = 1; i < count; i++)
+        if (a.job[i].kind != k) return k_flinear;
+    return k == KIND_F32 ? k_flinear_rows<KIND_F32> : (k == KIND_BF16 ? k_flinear_rows<KIND_BF16> : k_flinear);
 }
 
-// Workgroups of a linear kernel resident per CU at `lds` dynamic bytes
+// Workgroups of an F32 / BF16 kernel resident per CU at `lds` dynamic bytes
 // (occupancy query, cached per kernel and size).
 int fl_resident(const void* kern, size_t lds) {
     struct Entry {
@@ -710,104 +1268,63 @@ int fl_resident(const void* kern, size_t lds) {
 }
 
 size_t stage_bytes(uint32_t kind, int n) {
-    return (kind == KIND_F32 || kind == KIND_BF16) ? 4 * (size_t)n : (size_t)NLIMB * n + 4 * (size_t)(n / 32);
+    if (kind == KIND_F32 || kind == KIND_BF16) return 4 * (size_t)n;
+    const size_t ng = ((size_t)n + XGROUP - 1) / XGROUP;
+    return (XCHUNK * (XGROUP / 16) + 8) * ng;
 }
 
-int wave_rows(uint32_t kind) {
+// Instructions of a wave for 16 rows per column, and of the staging per column,
+// relative to each other.
+constexpr double STAGE_COST = 0.55;  // about 130 instructions per 256 columns against 190 for a step of them
+double step_cost(uint32_t kind) {
     switch (kind) {
-    case KIND_F32: return rows_per_wave<FK<KIND_F32>>();
-    case KIND_BF16: return rows_per_wave<FK<KIND_BF16>>();
-    case KIND_Q8_0: return rows_per_wave<FK<KIND_Q8_0>>();
-    case KIND_IQ4_NL: return rows_per_wave<FK<KIND_IQ4_NL>>();
-    case KIND_IQ4_XS: return rows_per_wave<FK<KIND_IQ4_XS>>();
-    case KIND_Q6_K: return rows_per_wave<FK<KIND_Q6_K>>();
-    case KIND_IQ3_XXS: return rows_per_wave<FK<KIND_IQ3_XXS>>();
+    case KIND_Q8_0: return 0.5;
+    case KIND_IQ4_NL: return 1.1;
     }
-    return 0;
+    return 0.9;
 }
+// Tiles whose segments meet at once: 32 KB of LDS, one where x takes more than
+// 64 KB (n > 7168), so that the largest x (149 KB) still fits.
+constexpr int FL_DEP = 4;
 
-bool linear_kind(uint32_t kind) { return wave_rows(kind) > 0; }
+bool row_kind(uint32_t kind) { return kind == KIND_F32 || kind == KIND_BF16; }
 
-}  // namespace
-
-// Plane layout of an uploaded frontier kind (the Q8_0 split is the matvec's:
-// int8 plane + fp16 plane). Returns false for kinds without one.
-bool frontier_layout(uint32_t kind, FrontierLayout& L) {
-    std::memset(&L, 0, sizeof(L));
-    auto put = [&](int o, int plane, int off) { L.map[o] = (uint16_t)((plane << 12) | off); };
+bool linear_kind(uint32_t kind) {
     switch (kind) {
     case KIND_F32:
     case KIND_BF16:
-        // 16-byte blocks copied as they are (n % 8 == 0)
-        L.block_vals = kind == KIND_F32 ? 4 : 8;
-        L.block_bytes = 16;
-        L.plane_bytes[0] = 16;
-        for (int o = 0; o < 16; o++) put(o, 0, o);
-        return true;
+    case KIND_Q8_0:
     case KIND_IQ4_NL:
-        L.block_vals = 32;
-        L.block_bytes = 18;
-        L.plane_bytes[0] = 16;
-        L.plane_bytes[2] = 2;
-        put(0, 2, 0);
-        put(1, 2, 1);
-        for (int o = 2; o < 18; o++) put(o, 0, o - 2);
-        return true;
     case KIND_IQ4_XS:
-        L.block_vals = 256;
-        L.block_bytes = 136;
-        L.plane_bytes[0] = 128;
-        L.plane_bytes[1] = 8;
-        for (int o = 0; o < 8; o++) put(o, 1, o);
-        for (int o = 8; o < 136; o++) put(o, 0, o - 8);
-        return true;
     case KIND_Q6_K:
-        L.block_vals = 256;
-        L.block_bytes = 210;
-        L.plane_bytes[0] = 192;
-        L.plane_bytes[1] = 16;
-        L.plane_bytes[2] = 2;
-        for (int o = 0; o < 128; o++) {  // ql
-            const int sub = o / 64, r = o % 64, half = r / 32, h = (r % 32) / 16, t = r % 16;
-            put(o, 0, 48 * (2 * sub + h) + 16 * half + t);
-        }
-        for (int o = 128; o < 192; o++) {  // qh
-            const int r = o - 128, sub = r / 32, h = (r % 32) / 16, t = r % 16;
-            put(o, 0, 48 * (2 * sub + h) + 32 + t);
-        }
-        for (int o = 192; o < 208; o++) {  // scales: byte sub*8 + h + 2g -> unit 2*sub+h, slot g
-            const int i = o - 192, sub = i / 8, w = i % 8, h = w % 2, g = w / 2;
-            put(o, 1, 4 * (2 * sub + h) + g);
-        }
-        put(208, 2, 0);
-        put(209, 2, 1);
-        return true;
-    case KIND_IQ3_XXS:
-        L.block_vals = 256;
-        L.block_bytes = 98;
-        L.plane_bytes[0] = 96;
-        L.plane_bytes[2] = 2;
-        put(0, 2, 0);
-        put(1, 2, 1);
-        for (int o = 2; o < 66; o++) {  // grid indices
-            const int r = o - 2;
-            put(o, 0, 48 * (r / 32) + r % 32);
-        }
-        for (int o = 66; o < 98; o++) {  // sign/scale words
-            const int r = o - 66;
-            put(o, 0, 48 * (r / 16) + 32 + r % 16);
-        }
-        return true;
+    case KIND_IQ3_XXS: return true;
     }
     return false;
 }
 
-static MapArgs map_args(const FrontierLayout& L) {
-    MapArgs a;
-    std::memcpy(a.map, L.map, sizeof(a.map));
-    a.block_bytes = L.block_bytes;
-    for (int i = 0; i < 3; i++) a.plane_bytes[i] = L.plane_bytes[i];
-    return a;
+}  // namespace
+
+// Device layout of an uploaded frontier kind (the Q8_0 split is the matvec's:
+// int8 plane + fp16 plane). Returns false for kinds without one.
+bool frontier_layout(uint32_t kind, FrontierLayout& L) {
+    L = FrontierLayout{};
+    switch (kind) {
+    case KIND_F32: L = {4, 16, 0, {}}; return true;
+    case KIND_BF16: L = {8, 16, 0, {}}; return true;
+    // lane group g: block 4t + g of step t, its scale in the lane plane
+    case KIND_IQ4_NL: L = {32, 18, 128, {1024, 128, 0}}; return true;
+    // lane group g: blocks g and 4 + g; row plane: 8 scale bytes of 16 rows, their d
+    case KIND_IQ4_XS: L = {256, 136, 256, {2048, 0, 160}}; return true;
+    case KIND_IQ3_XXS: L = {256, 98, 256, {2048, 0, 160}}; return true;
+    // lane group g = 2*sub + h: its three 16-byte pieces and, in the lane plane, four scales
+    case KIND_Q6_K: L = {256, 210, 256, {3072, 256, 32}}; return true;
+    }
+    return false;
+}
+
+size_t frontier_plane_bytes(const FrontierLayout& L, int plane, int64_t n, int64_t m) {
+    if (!L.step_vals) return plane == FL_BODY ? (size_t)(n / L.block_vals * m) * L.block_bytes : 0;
+    return (size_t)((m + 15) / 16) * ((n + L.step_vals - 1) / L.step_vals) * L.rec[plane];
 }
 
 static int grid_blocks(int64_t total) {
@@ -815,16 +1332,32 @@ static int grid_blocks(int64_t total) {
     return (int)std::min<int64_t>(std::max<int64_t>(g, 1), 65536);
 }
 
-void launch_layout_repack(const uint8_t* src, int64_t blocks, const FrontierLayout& L, uint8_t* const planes[3],
-                          hipStream_t s) {
-    hipLaunchKernelGGL(k_layout_repack, dim3(grid_blocks(blocks * L.block_bytes)), dim3(FWG), 0, s, src, blocks,
-                       map_args(L), planes[0], planes[1], planes[2]);
-}
-
-void launch_layout_verify(const uint8_t* src, int64_t blocks, const FrontierLayout& L, uint8_t* const planes[3],
-                          unsigned* bad, hipStream_t s) {
-    hipLaunchKernelGGL(k_layout_verify, dim3(grid_blocks(blocks * L.block_bytes)), dim3(FWG), 0, s, src, blocks,
-                       map_args(L), planes[0], planes[1], planes[2], bad);
+void launch_layout(uint32_t kind, const uint8_t* src, int64_t n, int64_t m, const FrontierLayout& L,
+                   uint8_t* const planes[3], unsigned* bad, hipStream_t s) {
+    const int64_t total = n / L.block_vals * m * L.block_bytes;
+    if (!L.step_vals) {
+        (void)hipMemcpyAsync(planes[FL_BODY], src, (size_t)total, hipMemcpyDeviceToDevice, s);
+        hipLaunchKernelGGL(k_copy_verify, dim3(grid_blocks(total / 16)), dim3(FWG), 0, s, (const uint4*)src,
+                           (const uint4*)planes[FL_BODY], total / 16, bad);
+        return;
+    }
+    LayoutArgs a{};
+    a.m = m;
+    a.kind = (int32_t)kind;
+    a.block_bytes = L.block_bytes;
+    a.blocks = (int32_t)(n / L.block_vals);
+    a.steps = (int32_t)((n + L.step_vals - 1) / L.step_vals);
+    a.bps = L.step_vals / L.block_vals;
+    for (int i = 0; i < 3; i++) {
+        a.rec[i] = L.rec[i];
+        a.plane[i] = planes[i];
+    }
+    for (int i = 0; i < 3; i++)
+        if (L.rec[i]) {
+            const int64_t dwords = (int64_t)frontier_plane_bytes(L, i, n, m) / 4;
+            hipLaunchKernelGGL(k_layout_repack, dim3(grid_blocks(dwords)), dim3(FWG), 0, s, src, a, i, dwords);
+        }
+    hipLaunchKernelGGL(k_layout_verify, dim3(grid_blocks(total)), dim3(FWG), 0, s, src, a, total, bad);
 }
 
 }  // namespace uq
@@ -836,8 +1369,8 @@ namespace {
 FJob make_job(const Weight& w, const float* x, float* y) {
     FJob j{};
     j.body = (const uint8_t*)w.qs;
-    j.aux = w.sc;
-    j.d = w.d;
+    j.lane = w.sc;
+    j.row = (const uint8_t*)w.d;
     j.x = x;
     j.y = y;
     j.m = w.m;
@@ -847,10 +1380,6 @@ FJob make_job(const Weight& w, const float* x, float* y) {
     case KIND_F32: j.pitch = 4 * w.n; break;
     case KIND_BF16: j.pitch = 2 * w.n; break;
     case KIND_Q8_0: j.pitch = w.n; break;
-    case KIND_IQ4_NL:
-    case KIND_IQ4_XS: j.pitch = w.n / 2; break;
-    case KIND_Q6_K: j.pitch = w.n / 256 * 192; break;
-    case KIND_IQ3_XXS: j.pitch = w.n / 256 * 96; break;
     }
     return j;
 }
@@ -871,48 +1400,106 @@ int enqueue_jobs(const uq_linear_job* jobs, int count, hipStream_t s) {
         if ((uintptr_t)jobs[i].x & 15) return set_error(ERR_ARG, "linear: x must be 16-byte aligned");
     }
     for (int c0 = 0; c0 < count; c0 += MAX_JOBS) {
-        JobArgs a{};
-        a.count = std::min(MAX_JOBS, count - c0);
+        JobArgs a;
+        const int jobs_here = std::min(MAX_JOBS, count - c0);
         size_t lds = 0;
-        for (int i = 0; i < a.count; i++) {
+        bool rows_only = true;
+        for (int i = 0; i < jobs_here; i++) {
             const Weight& w = jobs[c0 + i].weight->w;
             a.job[i] = make_job(w, jobs[c0 + i].x, jobs[c0 + i].y);
             lds = std::max(lds, stage_bytes(w.kind, (int)w.n));
+            rows_only = rows_only && row_kind(w.kind);
         }
-        // each job gets at most as many workgroups as fit on the chip at once
-        // (every workgroup loops over its row blocks); a table that cannot fill
-        // the chip with 512-thread workgroups runs 256-thread ones, twice as many
-        const FlKernel kern = kernel_for(a);
+        const bool one = jobs_here == 1;
         const int64_t cu = cu_count();
-        int threads = FL_WG;
         int64_t wg = 0;
-        for (int pass = 0; pass < 2; pass++) {
-            const int64_t cap = cu * fl_resident((const void*)kern, lds) * (FL_WG / threads);
-            wg = 0;
-            for (int i = 0; i < a.count; i++) {
-                const Weight& w = jobs[c0 + i].weight->w;
-                const int64_t rpb = (int64_t)wave_rows(w.kind) * (threads / 64);
-                const int64_t rblocks = (w.m + rpb - 1) / rpb;
-                a.job[i].wg0 = (int32_t)wg;
-                a.job[i].wgs = (int32_t)std::min<int64_t>(rblocks, cap);
-                wg += a.job[i].wgs;
+        int threads = FL_WG;
+        bool few = false;
+        if (!rows_only) {
+            // Tiles per workgroup, from those that make one to four workgroups a
+            // CU: the fewest instructions that a CU runs one behind the other, the
+            // staging of x in every workgroup among them. One workgroup a CU (two
+            // waves per SIMD) leaves some of its time idle.
+            int64_t tiles = 0;
+            for (int i = 0; i < jobs_here; i++)
+                if (!row_kind((uint32_t)a.job[i].kind)) tiles += (a.job[i].m + 15) / 16;
+            int64_t best = 0;
+            double least = 0.0;
+            for (int c = 0; c < 8; c++) {
+                const int64_t nt = (tiles + (c / 2 + 1) * cu - 1) / ((c / 2 + 1) * cu) + (c & 1);
+                int64_t wgs = 0;
+                double work = 0.0;
+                for (int i = 0; i < jobs_here; i++) {
+                    const FJob& j = a.job[i];
+                    const int64_t w = row_kind((uint32_t)j.kind) ? (j.m + 7) / 8 : ((j.m + 15) / 16 + nt - 1) / nt;
+                    wgs += w;
+                    work += (double)w * ((double)nt * step_cost((uint32_t)j.kind) + STAGE_COST) * j.n;
+                }
+                const int64_t per_cu = (wgs + cu - 1) / cu;
+                const double cost = work / (double)wgs * (double)per_cu * (per_cu == 1 ? 1.1 : 1.0);
+                if (!best || cost < least) {
+                    best = nt;
+                    least = cost;
+                }
             }
-            if (pass == 0 && wg < 2 * cu) threads = FL_WG / 2;
-            else break;
+            const int64_t step_vals = a.job[0].kind == KIND_Q8_0 || a.job[0].kind == KIND_IQ4_NL ? 128 : 256;
+            few = best * ((a.job[0].n + step_vals - 1) / step_vals) <= 2 * FL_SEGS;
+            for (int i = 0; i < jobs_here; i++) {
+                FJob& j = a.job[i];
+                j.wg0 = (int32_t)wg;
+                j.wgs = (int32_t)(row_kind((uint32_t)j.kind) ? std::min<int64_t>((j.m + 7) / 8, 4 * cu)
+                                                             : ((j.m + 15) / 16 + best - 1) / best);
+                wg += j.wgs;
+            }
+            a.parts.at = (int)((lds + 15) & ~(size_t)15);
+            a.parts.dep = a.parts.at <= 64 * 1024 ? FL_DEP : 1;
+            lds = (size_t)a.parts.at + 2 * 8 * 64 * FL_SEGS * (size_t)a.parts.dep;
+        } else {
+            // F32 / BF16: as many workgroups as fit on the chip at once; where
+            // 512-thread ones cannot fill it, 256-thread ones, twice as many
+            for (int pass = 0; pass < 2; pass++) {
+                const void* const kern = one ? (const void*)one_kernel(a.job[0].kind, false) : (const void*)table_kernel(a, jobs_here);
+                const int64_t cap = cu * fl_resident(kern, lds) * (FL_WG / threads), rpb = threads / 64;
+                wg = 0;
+                for (int i = 0; i < jobs_here; i++) {
+                    a.job[i].wg0 = (int32_t)wg;
+                    a.job[i].wgs = (int32_t)std::min<int64_t>((a.job[i].m + rpb - 1) / rpb, cap);
+                    wg += a.job[i].wgs;
+                }
+                if (pass == 0 && wg < 2 * cu) threads = FL_WG / 2;
+                else break;
+            }
         }
         if (wg > 0x7fffffff) return set_error(ERR_SHAPE, "linear: job table too large for one launch");
         static bool lds_set = false;
         if (!lds_set) {
-            const FlKernel all[] = {k_flinear, k_flinear_kind<KIND_F32>, k_flinear_kind<KIND_BF16>,
-                                    k_flinear_kind<KIND_Q8_0>, k_flinear_kind<KIND_IQ4_NL>,
-                                    k_flinear_kind<KIND_IQ4_XS>, k_flinear_kind<KIND_Q6_K>,
-                                    k_flinear_kind<KIND_IQ3_XXS>};
-            for (FlKernel f : all)
-                UQ_CHECK_HIP(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 (int)stage_bytes(KIND_Q8_0, 16384)));
+            const void* const all[] = {
+                (const void*)k_flinear, (const void*)k_flinear_rows<KIND_F32>, (const void*)k_flinear_rows<KIND_BF16>,
+                (const void*)k_flinear_one<KIND_F32>, (const void*)k_flinear_one<KIND_BF16>,
+                (const void*)k_flinear_one<KIND_Q8_0>, (const void*)k_flinear_one<KIND_Q8_0, 1>,
+                (const void*)k_flinear_one<KIND_IQ4_NL>, (const void*)k_flinear_one<KIND_Q6_K, 1>,
+                (const void*)k_flinear_one<KIND_IQ4_XS>, (const void*)k_flinear_one<KIND_Q6_K>,
+                (const void*)k_flinear_one<KIND_IQ3_XXS>};
+            for (const void* f : all)
+                UQ_CHECK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)(stage_bytes(KIND_Q8_0, 16384) + 16 * 64 * FL_SEGS)));
             lds_set = true;
         }
-        hipLaunchKernelGGL(kern, dim3((unsigned)wg), dim3(threads), lds, s, a);
+        if (one) {
+            hipLaunchKernelGGL(one_kernel(a.job[0].kind, few), dim3((unsigned)wg), dim3(threads), lds, s,
+                               (OneJob{a.parts, a.job[0]}));
+        } else {
+            int64_t widest = 0;
+            for (int i = 0; i < MAX_JOBS; i++) {
+                a.start[i] = i < jobs_here ? a.job[i].wg0 : 0x7fffffff;
+                if (i < jobs_here) widest = std::max<int64_t>(widest, a.job[i].wgs);
+            }
+            // a grid row per job, as wide as the widest, unless that leaves more
+            // than half of the workgroups without work
+            const bool rows = widest * jobs_here <= 2 * wg;
+            const dim3 grid = rows ? dim3((unsigned)widest, (unsigned)jobs_here) : dim3((unsigned)wg);
+            hipLaunchKernelGGL(table_kernel(a, jobs_here), grid, dim3(threads), lds, s, a);
+        }
         UQ_CHECK_HIP(hipGetLastError());
     }
     return OK;

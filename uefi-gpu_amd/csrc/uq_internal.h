@@ -43,8 +43,8 @@ int set_error(int status, const std::string& msg);
 int64_t row_bytes(uint32_t kind, int64_t n);  // GGUF bytes of one row, <0 if invalid
 
 // Device-resident weight. The frontier kinds (F32, BF16, Q6_K, IQ3_XXS,
-// IQ4_NL, IQ4_XS) use the planes of their FrontierLayout: qs = body units,
-// sc = aux bytes, d = fp16 block scales. Q8_0 is split into an int8 plane qs[m][n] and an
+// IQ4_NL, IQ4_XS) use the planes of their FrontierLayout: qs = body,
+// sc = lane records, d = row records. Q8_0 is split into an int8 plane qs[m][n] and an
 // fp16 scale plane d[m][n/32]; Q4_K and Q3_K use the unit planes of Q4K /
 // Q3K (qs, sc, d); lm_head-sized Q3_K weights use the row-block layout of
 // Q3KSB in qs alone.
@@ -72,19 +72,23 @@ int staging_buffer(size_t bytes, void** out);
 
 int upload_weight(uint32_t kind, int64_t n, int64_t m, const void* gguf, size_t bytes, Weight& out, bool bank);
 
-// Split of one GGUF block of a frontier kind into three planes (body, aux,
-// fp16 scale): map[o] = plane << 12 | offset of source byte o within that
-// plane's per-block slice of plane_bytes[plane] bytes (uq_frontier.hip).
+// Device layout of a frontier kind (uq_frontier.hip). F32 and BF16 rows stay as
+// they are (step_vals 0). The others are cut into tiles of 16 rows and steps of
+// step_vals columns, in the order in which a wave reads them; rec[] = bytes of a
+// tile's step in each plane: the body plane holds pieces of 64 lanes x 16 bytes,
+// the lane plane a record per lane, the row plane one per row; lane 16*g + r
+// serves row r. Rows past the last and columns past n are zero.
+enum FrontierPlane { FL_BODY = 0, FL_LANE = 1, FL_ROW = 2 };
 struct FrontierLayout {
-    int block_vals, block_bytes;
-    int plane_bytes[3];
-    uint16_t map[256];
+    int block_vals, block_bytes, step_vals;
+    int rec[3];
 };
 bool frontier_layout(uint32_t kind, FrontierLayout& L);
-void launch_layout_repack(const uint8_t* src, int64_t blocks, const FrontierLayout& L, uint8_t* const planes[3],
-                          hipStream_t s);
-void launch_layout_verify(const uint8_t* src, int64_t blocks, const FrontierLayout& L, uint8_t* const planes[3],
-                          unsigned* bad, hipStream_t s);
+size_t frontier_plane_bytes(const FrontierLayout& L, int plane, int64_t n, int64_t m);
+// Repacks GGUF rows into the planes, then rebuilds every GGUF byte from them and
+// adds the number of differing ones to *bad.
+void launch_layout(uint32_t kind, const uint8_t* src, int64_t n, int64_t m, const FrontierLayout& L,
+                   uint8_t* const planes[3], unsigned* bad, hipStream_t s);
 
 // ---- kernel launchers (uq_matvec.hip) ----
 void launch_quant_act(const float* x, int64_t n, int8_t* xq, float* xs, hipStream_t s);

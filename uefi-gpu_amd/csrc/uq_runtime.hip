@@ -186,11 +186,11 @@ namespace uq {
 static int upload_split(uint32_t kind, int64_t n, int64_t m, const void* gguf, int64_t rb, const FrontierLayout& L,
                         Weight& out) {
     hipStream_t s = g_ctx.stream;
-    const int64_t blocks = n / L.block_vals * m;
-    size_t off[3], total = 0;
+    size_t off[3], len[3], total = 0;
     for (int p = 0; p < 3; p++) {
         off[p] = total;
-        total += align256((size_t)(blocks * L.plane_bytes[p]));
+        len[p] = frontier_plane_bytes(L, p, n, m);
+        total += align256(len[p]);
     }
     Weight w;
     w.kind = kind;
@@ -202,15 +202,14 @@ static int upload_split(uint32_t kind, int64_t n, int64_t m, const void* gguf, i
     uint8_t* base = (uint8_t*)w.alloc;
     uint8_t* planes[3] = {base + off[0], base + off[1], base + off[2]};
     w.qs = (const int8_t*)planes[0];
-    w.sc = L.plane_bytes[1] ? planes[1] : nullptr;
-    w.d = L.plane_bytes[2] ? (const uint16_t*)planes[2] : nullptr;
+    w.sc = len[FL_LANE] ? planes[FL_LANE] : nullptr;
+    w.d = len[FL_ROW] ? (const uint16_t*)planes[FL_ROW] : nullptr;
     void* staging = nullptr;
     hipError_t e = hipMalloc(&staging, (size_t)w.gguf_bytes);
     if (e == hipSuccess) e = hipMemcpyAsync(staging, gguf, (size_t)w.gguf_bytes, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemsetAsync(g_ctx.dcount, 0, sizeof(unsigned), s);
     if (e == hipSuccess) {
-        launch_layout_repack((const uint8_t*)staging, blocks, L, planes, s);
-        launch_layout_verify((const uint8_t*)staging, blocks, L, planes, g_ctx.dcount, s);
+        launch_layout(kind, (const uint8_t*)staging, n, m, L, planes, g_ctx.dcount, s);
         e = hipGetLastError();
     }
     unsigned bad = 0;

@@ -1505,12 +1505,6 @@ int enqueue_jobs(const uq_linear_job* jobs, int count, hipStream_t s) {
     return OK;
 }
 
-int check_finite(const float* v, int64_t n, const char* what) {
-    for (int64_t i = 0; i < n; i++)
-        if (!std::isfinite(v[i])) return set_error(ERR_NONFINITE, std::string(what) + ": non-finite value");
-    return OK;
-}
-
 }  // namespace
 
 
@@ -1561,40 +1555,47 @@ int uq_linear_batch(const uq_linear_job* jobs, int count) {
         xs += jobs[i].weight->w.n;
         ys += jobs[i].weight->w.m;
     }
-    for (int i = 0; i < count; i++)
-        if (int rc = check_finite(jobs[i].x, jobs[i].weight->w.n, "linear_batch: input")) return rc;
     hipStream_t s = (hipStream_t)uq_stream();
     const size_t x_bytes = (sizeof(float) * (size_t)xs + 255) & ~(size_t)255;
-    void* stage = nullptr;
-    if (int rc = staging_buffer(x_bytes + sizeof(float) * (size_t)ys, &stage)) return rc;
-    float* const dx = (float*)stage;
-    float* const dy = (float*)((char*)stage + x_bytes);
-    hipError_t e = hipSuccess;
-    int rc = OK;
-    std::vector<uq_linear_job> dj((size_t)count);
-    std::vector<float> host((size_t)ys);
+    void *stage = nullptr, *host = nullptr;
+    if (int rc = host_buffer(x_bytes + sizeof(float) * (size_t)ys + 16, &host)) return rc;
+    float* const hx = (float*)host;
+    float* const hy = (float*)((char*)host + x_bytes);
     int64_t xo = 0, yo = 0;
-    for (int i = 0; i < count && e == hipSuccess; i++) {
+    for (int i = 0; i < count; i++) {
+        const int64_t n = jobs[i].weight->w.n;
+        if (!copy_finite(hx + xo, jobs[i].x, n)) return set_error(ERR_NONFINITE, "linear_batch: input: non-finite value");
+        xo += n;  // n % 8 == 0 keeps every x 32-byte aligned
+    }
+    const bool direct = ys <= HOST_DIRECT;
+    if (int rc = staging_buffer(x_bytes + (direct ? 0 : sizeof(float) * (size_t)ys + 16), &stage)) return rc;
+    float* const dx = (float*)stage;  // every workgroup of a job reads its x
+    float* const dy = direct ? hy : (float*)((char*)stage + x_bytes);
+    std::vector<uq_linear_job> dj((size_t)count);
+    xo = 0;
+    for (int i = 0; i < count; i++) {
         const Weight& w = jobs[i].weight->w;
-        e = hipMemcpyAsync(dx + xo, jobs[i].x, sizeof(float) * (size_t)w.n, hipMemcpyHostToDevice, s);
         dj[(size_t)i] = uq_linear_job{jobs[i].weight, dx + xo, dy + yo};
-        xo += w.n;  // n % 8 == 0 keeps every x 32-byte aligned
+        xo += w.n;
         yo += w.m;
     }
-    if (e == hipSuccess) rc = enqueue_jobs(dj.data(), count, s);
-    if (e == hipSuccess && rc == OK)
-        e = hipMemcpyAsync(host.data(), dy, sizeof(float) * (size_t)ys, hipMemcpyDeviceToHost, s);
-    // a failed enqueue still leaves the copies above reading the staging buffer
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    launch_copy(dx, hx, sizeof(float) * (size_t)xs, s);
+    const int rc = enqueue_jobs(dj.data(), count, s);
+    if (rc == OK && !direct) launch_copy(hy, dy, sizeof(float) * (size_t)ys, s);
+    hipError_t e = hipGetLastError();
+    // a failed enqueue still leaves the copy above reading the pinned buffer
+    const hipError_t es = wait_host();
+    if (e == hipSuccess) e = es;
     if (e != hipSuccess) return set_error(ERR_DEVICE, std::string("linear_batch: ") + hipGetErrorString(e));
     if (rc != OK) return rc;
     yo = 0;
+    bool finite = true;
     for (int i = 0; i < count; i++) {
         const int64_t m = jobs[i].weight->w.m;
-        std::memcpy(jobs[i].y, host.data() + yo, sizeof(float) * (size_t)m);
+        finite = copy_finite(jobs[i].y, hy + yo, m) && finite;
         yo += m;
     }
-    return check_finite(host.data(), ys, "linear_batch: output");
+    return finite ? OK : set_error(ERR_NONFINITE, "linear_batch: output: non-finite value");
 }
 
 int uq_time_linear(const uq_weight_t* ws, int count, int reps, int warmup, double* total_ms) {

@@ -69,6 +69,16 @@ int cu_count();
 // grown on demand and never shrunk, so repeated calls of the same sizes
 // allocate nothing. Valid until the next call that asks for more bytes.
 int staging_buffer(size_t bytes, void** out);
+// Pinned host memory of the host-pointer linears, on the same terms.
+int host_buffer(size_t bytes, void** out);
+// Copies n values; false if one of them is not finite.
+bool copy_finite(float* dst, const float* src, int64_t n);
+// Waits for the work on the library stream.
+hipError_t wait_host();
+void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
+// Outputs of up to this many floats are stored to pinned memory by the linear
+// kernels themselves (4-byte stores over PCIe); larger ones are copied there.
+constexpr int64_t HOST_DIRECT = 2048;
 
 int upload_weight(uint32_t kind, int64_t n, int64_t m, const void* gguf, size_t bytes, Weight& out, bool bank);
 

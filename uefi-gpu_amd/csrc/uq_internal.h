@@ -118,6 +118,9 @@ void launch_sb_repack(uint32_t kind, const uint8_t* gguf, int64_t n, int64_t m, 
                       unsigned* bad, hipStream_t s);
 // y[m] = W x for any kind; gate/up fusion writes silu(gate)*up when w2 != null.
 int launch_matvec(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s);
+// y = W quant(x) from an f32 x, as launch_quant_act and launch_matvec give it bit
+// for bit, in one launch where that is faster; xq, xs: scratch of the other case.
+int launch_matvec_x(const Weight& w, const float* x, float* y, int8_t* xq, float* xs, hipStream_t s);
 int launch_block_dots(const Weight& w, const int8_t* xq, int32_t* dots, hipStream_t s);
 // Up to 8 Q8_0 weights of one input length (w2s[i] non-null: gate/up pair) in
 // one launch over a shared quantized x; each output as launch_matvec gives it.

@@ -264,6 +264,81 @@ __device__ __forceinline__ void matvec_row(const WArgs& w, const WArgs& w2, cons
     if (row < end && sub == 0) y[row] = GATEUP ? uq_silu_mul((float)acc, (float)acc2) : (float)acc;
 }
 
+// The activation quantized by the workgroup itself (the codes and scales of
+// k_quant_act): 4 values per thread and round, 8 threads to a 32-block.
+// put(q, codes, sum) gets the codes of values 4q .. 4q + 3 and the sum of the
+// 16-value group they lie in; scale(b, s) the scale of 32-block b. The chain
+// load, amax, division, code bounds it, not the 4K bytes read out of the L2: 4
+// rounds' loads go out together and their divisions are shared out over the 8
+// threads (K = 16384, few rows: 8.5 us with one round at a time, 6.9 with the
+// loads together, 6.0 with the divisions shared). x is 16-byte aligned.
+template <class P, class S>
+UQ_DEV void quant_x(const float* __restrict__ x, int64_t K, P&& put, S&& scale) {
+    constexpr int R = 4;
+    const int nq = (int)(K / 4), step = (int)blockDim.x;
+    for (int q0 = threadIdx.x; q0 < nq; q0 += R * step) {
+        float4 f[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int q = q0 + r * step;
+            f[r] = ((const float4*)x)[q < nq ? q : nq - 1];  // clamped: one fetch for all rounds
+        }
+        float amax[R], inv[R], sc[1];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            amax[r] = uq_group_max<8>(fmaxf(fmaxf(fabsf(f[r].x), fabsf(f[r].y)), fmaxf(fabsf(f[r].z), fabsf(f[r].w))));
+        uq_block_recips<R, 8>(amax, inv, sc);
+        const int lr = threadIdx.x & 7, qs = q0 + lr * step;
+        if (lr < R && qs < nq) scale(qs >> 3, sc[0]);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int q = q0 + r * step;
+            if (q >= nq) break;  // K % 32 == 0: the 8 threads of a block are all in or all out
+            const uint32_t codes = uq_quant_code(f[r].x, inv[r]) | uq_quant_code(f[r].y, inv[r]) << 8 |
+                                   uq_quant_code(f[r].z, inv[r]) << 16 | uq_quant_code(f[r].w, inv[r]) << 24;
+            int sum = uq_dot4(0x01010101, (int)codes, 0);
+            sum += uq_dpp<UQ_DPP_XOR1>(sum);
+            sum += uq_dpp<UQ_DPP_XOR2>(sum);
+            put(q, codes, sum);
+        }
+    }
+}
+
+// y = W x with the quantization of x in the same launch. Bound by the launch and
+// the chain of one workgroup until the weights outweigh them: the rows' weights
+// are requested first and arrive while x is quantized into LDS.
+template <class KQ, int LPR, int NBL>
+__global__ __launch_bounds__(WG) void k_matvec_f(WArgs w, const float* __restrict__ x, float* __restrict__ y,
+                                                 int64_t rows, int64_t K, int64_t share) {
+    constexpr int RPW = 64 / LPR, RPB = RPW * (WG / 64), MAXK = LPR * NBL * KQ::UNIT;
+    __shared__ __attribute__((aligned(16))) int8_t lq[MAXK];
+    __shared__ float ls[MAXK / 32 + 1];
+    const int64_t nu = K / KQ::UNIT;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane % LPR, grp = lane / LPR;
+    const RowSpan sp = even_span(rows, share);  // the grid covers the rows in one pass
+    const int64_t row = sp.begin + wave * RPW + grp;
+    typename KQ::W wv[NBL];
+    const typename KQ::R rp = KQ::row_ptr(w, row < sp.end ? row : sp.end - 1, nu);
+#pragma unroll
+    for (int i = 0; i < NBL; i++) {
+        const int u = sub + LPR * i;
+        wv[i] = KQ::load_u(rp, u < nu ? u : (int)nu - 1);
+    }
+    quant_x(x, K, [&](int q, uint32_t codes, int) { *(uint32_t*)(lq + 4 * q) = codes; }, [&](int b, float s) { ls[b] = s; });
+    __syncthreads();
+    typename KQ::X xr[NBL];
+    load_xr<KQ, LPR, NBL>(xr, lq, ls, nu, sub);
+    double acc = 0.0;
+#pragma unroll
+    for (int i = 0; i < NBL; i++) {
+        const int u = sub + LPR * i, uc = u < nu ? u : (int)nu - 1;
+        const double t = KQ::dot(wv[i], xr[i], uc);
+        acc += u < nu ? t : 0.0;
+    }
+    acc = uq_group_sum<LPR>(acc);
+    if (row < sp.end && sub == 0) y[row] = (float)acc;
+}
+
 template <class KQ, int LPR, int NBL, bool GATEUP>
 __global__ __launch_bounds__(WG) void k_matvec(WArgs w, WArgs w2, const int8_t* __restrict__ xq,
                                                const float* __restrict__ xs, float* __restrict__ y,
@@ -374,11 +449,13 @@ __device__ __forceinline__ void matvec_row_lds(const WArgs& w, const WArgs& w2, 
 // registers across rows, so the workgroup stages the quantized activation,
 // its scales and its 16-value sums in LDS once and each unit reads its slice
 // from LDS right before its dot. K <= MAX_XL.
+// FX (uq_matvec_static): the workgroup quantizes x itself.
 constexpr int MAX_XL = 16384;
-template <class KQ, int LPR, int NBL, bool GATEUP>
+template <class KQ, int LPR, int NBL, bool GATEUP, bool FX = false>
 __global__ __launch_bounds__(WG) void k_matvec_xl(WArgs w, WArgs w2, const int8_t* __restrict__ xq,
                                                   const float* __restrict__ xs, float* __restrict__ y,
-                                                  int64_t rows, int64_t K, int64_t share) {
+                                                  int64_t rows, int64_t K, int64_t share,
+                                                  const float* __restrict__ x) {
     // dynamic LDS sized to K (xl_lds_bytes): x (K int8), its scales (K/32 f32), its 16-value sums (K/16
     // int, as KQ::stage16 forms them)
     extern __shared__ __attribute__((aligned(16))) int8_t xl_lds[];
@@ -390,16 +467,26 @@ __global__ __launch_bounds__(WG) void k_matvec_xl(WArgs w, WArgs w2, const int8_
     const int64_t nu = K / KQ::UNIT;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sub = lane % LPR, grp = lane / LPR;
-    for (int g = threadIdx.x; g < K / 16; g += WG) {
-        const int4 v = ((const int4*)xq)[g];
-        ((int4*)lx)[g] = v;
-        const int ones = 0x01010101;
-        int c = uq_dot4(ones, v.x, 0);
-        c = uq_dot4(ones, v.y, c);
-        c = uq_dot4(ones, v.z, c);
-        ls16[g] = KQ::stage16(g, uq_dot4(ones, v.w, c));
+    if constexpr (FX) {
+        quant_x(
+            x, K,
+            [&](int q, uint32_t codes, int sum) {
+                *(uint32_t*)(lx + 4 * q) = codes;
+                if ((q & 3) == 0) ls16[q >> 2] = KQ::stage16(q >> 2, sum);
+            },
+            [&](int b, float s) { lxs[b] = s; });
+    } else {
+        for (int g = threadIdx.x; g < K / 16; g += WG) {
+            const int4 v = ((const int4*)xq)[g];
+            ((int4*)lx)[g] = v;
+            const int ones = 0x01010101;
+            int c = uq_dot4(ones, v.x, 0);
+            c = uq_dot4(ones, v.y, c);
+            c = uq_dot4(ones, v.z, c);
+            ls16[g] = KQ::stage16(g, uq_dot4(ones, v.w, c));
+        }
+        for (int b = threadIdx.x; b < K / 32; b += WG) lxs[b] = xs[b];
     }
-    for (int b = threadIdx.x; b < K / 32; b += WG) lxs[b] = xs[b];
     __syncthreads();
     if (rows <= (int64_t)gridDim.x * RPB) {
         // one pass: this workgroup's even share of the rows
@@ -461,10 +548,11 @@ template <> struct SbDot<Q3KSB> {
     }
 };
 
-template <class KS, bool GATEUP>
+template <class KS, bool GATEUP, bool FX = false>
 __global__ __launch_bounds__(WG) void k_matvec_sb(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                                                   const int8_t* __restrict__ xq, const float* __restrict__ xs,
-                                                  float* __restrict__ y, int64_t rows, int64_t blocks, SbArgs g) {
+                                                  float* __restrict__ y, int64_t rows, int64_t blocks, SbArgs g,
+                                                  const float* __restrict__ x) {
     extern __shared__ __attribute__((aligned(16))) int8_t sb_lds[];
     constexpr int P = KS::P;
     const int S = g.S, LB = g.LB, RB = g.RB, K = 256 * S;
@@ -473,13 +561,23 @@ __global__ __launch_bounds__(WG) void k_matvec_sb(const uint8_t* __restrict__ w,
     int* l16 = (int*)(lxs + SB_XS * S);
     double* part = (double*)(l16 + SB_S16 * S);
     const int tid = threadIdx.x, nthr = blockDim.x, bpw = nthr / LB;
-    for (int gi = tid; gi < K / 16; gi += nthr) {
-        const int4 v = ((const int4*)xq)[gi];
-        const int sb = gi >> 4, wi = gi & 15;
-        *(int4*)(lx + sb * SB_X + 16 * wi) = v;
-        l16[sb * SB_S16 + wi] = SbDot<KS>::stage16(wi, Q3K::sum16(v));
+    if constexpr (FX) {
+        quant_x(
+            x, K,
+            [&](int q, uint32_t codes, int sum) {
+                *(uint32_t*)(lx + (q >> 6) * SB_X + 4 * (q & 63)) = codes;
+                if ((q & 3) == 0) l16[(q >> 6) * SB_S16 + ((q >> 2) & 15)] = SbDot<KS>::stage16((q >> 2) & 15, sum);
+            },
+            [&](int b, float s) { lxs[(b >> 3) * SB_XS + (b & 7)] = s; });
+    } else {
+        for (int gi = tid; gi < K / 16; gi += nthr) {
+            const int4 v = ((const int4*)xq)[gi];
+            const int sb = gi >> 4, wi = gi & 15;
+            *(int4*)(lx + sb * SB_X + 16 * wi) = v;
+            l16[sb * SB_S16 + wi] = SbDot<KS>::stage16(wi, Q3K::sum16(v));
+        }
+        for (int b = tid; b < K / 32; b += nthr) lxs[(b >> 3) * SB_XS + (b & 7)] = xs[b];
     }
-    for (int b = tid; b < K / 32; b += nthr) lxs[(b >> 3) * SB_XS + (b & 7)] = xs[b];
     __syncthreads();
     const int64_t blk = (int64_t)blockIdx.x * bpw + tid / LB;
     const int j = tid % LB, rr = j / S, s = j - rr * S;
@@ -619,13 +717,48 @@ int resident_blocks(const void* kern, size_t lds) {
     return n;
 }
 
+constexpr int TWO_LAUNCHES = 1;  // launch_kind's answer where x is better quantized by a launch of its own
+
+// Whether every one of g workgroups quantizing x costs less than a launch that
+// does it once: the saved launch and its gap are worth 2.1 us, one workgroup's
+// own quantization is a chain of some 0.25 us per 1024 values, and the work of
+// the workgroups that share a CU adds up. Measured over Q8_0, Q4_K and Q3_K,
+// K 512 .. 16384 and 256 .. 16000 workgroups (two launches -> one, us):
+//   K 512    g 256 6.3 -> 4.1   g 4000 8.5 -> 8.1     g 8000 12.9 -> 13.2
+//   K 1536   g 256 6.4 -> 4.2   g 4000 10.9 -> 10.7   g 8000 18.0 -> 19.1
+//   K 4096   g 256 6.4 -> 4.4   g 1024 7.7 -> 6.7     g 4000 13.7 -> 14.3
+//   K 8960   g 256 6.3 -> 5.7   g 512 7.0 -> 7.5      g 1024 8.4 -> 10.0
+//   K 16384  g 256 6.6 -> 6.8   g 512 8.6 -> 9.6
+// One launch won at every point below the line K (g + 1.5 CUs) = 29000 CUs and
+// lost or tied at all but a few above it.
+bool quant_pays(int64_t K, int64_t g) {
+    const int64_t cu = cu_count();
+    return K * (2 * g + 3 * cu) <= 58000 * cu;
+}
+
+// The register kernel's one-launch form. Only Q8_0's 16-value units take it: the
+// superblock kinds leave the LDS kernels past K = MAX_XL, where two launches win.
+template <class KQ, int LPR, int NBL>
+const void* fused_kernel() {
+    if constexpr (KQ::UNIT < 64) return (const void*)k_matvec_f<KQ, LPR, NBL>;
+    return nullptr;
+}
+
+// x != nullptr: the activation as f32, quantized in the same launch; false
+// where two launches are better (nothing has been launched then).
 template <class KQ, int LPR, int NBL, bool XL = false>
-void launch_t(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s) {
+bool launch_t(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s,
+              const float* x = nullptr) {
     constexpr int RPB = (64 / LPR) * (WG / 64);
     const size_t lds = XL ? xl_lds_bytes(w.n) : 0;
     const void* kern;
-    if constexpr (XL) kern = w2 ? (const void*)k_matvec_xl<KQ, LPR, NBL, true> : (const void*)k_matvec_xl<KQ, LPR, NBL, false>;
-    else kern = w2 ? (const void*)k_matvec<KQ, LPR, NBL, true> : (const void*)k_matvec<KQ, LPR, NBL, false>;
+    if constexpr (XL)
+        kern = x ? (const void*)k_matvec_xl<KQ, LPR, NBL, false, true>
+                 : (w2 ? (const void*)k_matvec_xl<KQ, LPR, NBL, true> : (const void*)k_matvec_xl<KQ, LPR, NBL, false>);
+    else
+        kern = x ? fused_kernel<KQ, LPR, NBL>()
+                 : (w2 ? (const void*)k_matvec<KQ, LPR, NBL, true> : (const void*)k_matvec<KQ, LPR, NBL, false>);
+    if (!kern) return false;
     // a multiple of the CU count with at most one pass of rows per workgroup
     // while that fits on the chip at once. Past that (lm_head), Q8_0 and Q4_K
     // take one row block per workgroup and leave the balancing to the
@@ -638,23 +771,28 @@ void launch_t(const Weight& w, const Weight* w2, const int8_t* xq, const float* 
     int64_t g = m * cu;
     if (g > fit) g = nblk;
     if (g > w.m) g = w.m;
+    if (x && !quant_pays(w.n, g)) return false;
     const unsigned grid = (unsigned)g;
     const int64_t share = w.m / g;
     WArgs a{w.qs, w.d, w.sc}, b{nullptr, nullptr, nullptr};
     if (w2) b = WArgs{w2->qs, w2->d, w2->sc};
     if constexpr (XL) {
-        if (w2) hipLaunchKernelGGL((k_matvec_xl<KQ, LPR, NBL, true>), dim3(grid), dim3(WG), lds, s, a, b, xq, xs, y, w.m, w.n, share);
-        else hipLaunchKernelGGL((k_matvec_xl<KQ, LPR, NBL, false>), dim3(grid), dim3(WG), lds, s, a, b, xq, xs, y, w.m, w.n, share);
+        if (x) hipLaunchKernelGGL((k_matvec_xl<KQ, LPR, NBL, false, true>), dim3(grid), dim3(WG), lds, s, a, b, xq, xs, y, w.m, w.n, share, x);
+        else if (w2) hipLaunchKernelGGL((k_matvec_xl<KQ, LPR, NBL, true>), dim3(grid), dim3(WG), lds, s, a, b, xq, xs, y, w.m, w.n, share, x);
+        else hipLaunchKernelGGL((k_matvec_xl<KQ, LPR, NBL, false>), dim3(grid), dim3(WG), lds, s, a, b, xq, xs, y, w.m, w.n, share, x);
     } else {
-        if (w2) hipLaunchKernelGGL((k_matvec<KQ, LPR, NBL, true>), dim3(grid), dim3(WG), 0, s, a, b, xq, xs, y, w.m, w.n, share);
+        if (x) ((void (*)(WArgs, const float*, float*, int64_t, int64_t, int64_t))kern)<<<dim3(grid), dim3(WG), 0, s>>>(a, x, y, w.m, w.n, share);
+        else if (w2) hipLaunchKernelGGL((k_matvec<KQ, LPR, NBL, true>), dim3(grid), dim3(WG), 0, s, a, b, xq, xs, y, w.m, w.n, share);
         else hipLaunchKernelGGL((k_matvec<KQ, LPR, NBL, false>), dim3(grid), dim3(WG), 0, s, a, b, xq, xs, y, w.m, w.n, share);
     }
+    return true;
 }
 
 // Row-block layout: one block per LB-lane group, the largest group count per
 // workgroup (of 256 threads at most) that still gives two workgroups per CU.
 template <class KS>
-int launch_sb(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s) {
+int launch_sb(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s,
+              const float* x = nullptr) {
     const SbGeom g = sb_geom(w.n, w.m);
     if (g.LB != w.sb_lb || g.RB != w.sb_rb || (w2 && (w2->sb_lb != w.sb_lb || w2->sb_rb != w.sb_rb)))
         return set_error(ERR_SHAPE, "matvec: row-block geometry differs from the upload's");
@@ -663,27 +801,32 @@ int launch_sb(const Weight& w, const Weight* w2, const int8_t* xq, const float* 
     const int nthr = bpw * g.LB;
     const unsigned grid = (unsigned)((g.blocks + bpw - 1) / bpw);
     const size_t lds = sb_lds_bytes(g.S, nthr, w2 != nullptr);
+    if (x && !quant_pays(w.n, grid)) return TWO_LAUNCHES;
     const SbArgs a{g.S, g.LB, g.RB};
     const uint8_t* q = (const uint8_t*)w.qs;
-    if (w2)
+    if (x)
+        hipLaunchKernelGGL((k_matvec_sb<KS, false, true>), dim3(grid), dim3(nthr), lds, s, q, nullptr, xq, xs, y, w.m,
+                           g.blocks, a, x);
+    else if (w2)
         hipLaunchKernelGGL((k_matvec_sb<KS, true>), dim3(grid), dim3(nthr), lds, s, q, (const uint8_t*)w2->qs, xq, xs, y,
-                           w.m, g.blocks, a);
+                           w.m, g.blocks, a, x);
     else
         hipLaunchKernelGGL((k_matvec_sb<KS, false>), dim3(grid), dim3(nthr), lds, s, q, nullptr, xq, xs, y, w.m,
-                           g.blocks, a);
+                           g.blocks, a, x);
     return OK;
 }
 
 // Lane-group size per row from the number of units per row: small rows use
 // short groups (more rows per wave), long rows spread over a full wave.
 template <class KQ>
-int launch_kind(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s) {
+int launch_kind(const Weight& w, const Weight* w2, const int8_t* xq, const float* xs, float* y, hipStream_t s,
+                const float* x = nullptr) {
     const int64_t nu = w.n / KQ::UNIT;
 #define UQ_TRY(L, B) \
-    if (nu <= (int64_t)(L) * (B)) { launch_t<KQ, L, B>(w, w2, xq, xs, y, s); return OK; }
+    if (nu <= (int64_t)(L) * (B)) return launch_t<KQ, L, B>(w, w2, xq, xs, y, s, x) ? OK : TWO_LAUNCHES;
     // K-quants: activation staged in LDS, lane groups sized to fit the row
 #define UQ_TRYX(L, B) \
-    if (nu <= (int64_t)(L) * (B)) { launch_t<KQ, L, B, true>(w, w2, xq, xs, y, s); return OK; }
+    if (nu <= (int64_t)(L) * (B)) return launch_t<KQ, L, B, true>(w, w2, xq, xs, y, s, x) ? OK : TWO_LAUNCHES;
     if constexpr (KQ::UNIT >= 64) {
         if (w.n <= MAX_XL) {
             UQ_TRYX(4, 1) UQ_TRYX(4, 2) UQ_TRYX(4, 3) UQ_TRYX(8, 3) UQ_TRYX(8, 4) UQ_TRYX(16, 3) UQ_TRYX(32, 3) UQ_TRYX(64, 3)
@@ -818,6 +961,24 @@ int launch_matvec(const Weight& w, const Weight* w2, const int8_t* xq, const flo
     case KIND_Q3_K: return w.sb_lb ? launch_sb<Q3KSB>(w, w2, xq, xs, y, s) : launch_kind<Q3K>(w, w2, xq, xs, y, s);
     default: return set_error(ERR_QUANT_TYPE, "matvec: unsupported kind");
     }
+}
+
+int launch_matvec_x(const Weight& w, const float* x, float* y, int8_t* xq, float* xs, hipStream_t s) {
+    // (y may lie over x where x has a launch of its own to be read in)
+    const bool apart = y + w.m <= x || x + w.n <= y;
+    if (apart && ((uintptr_t)x & 15) == 0) {
+        int rc = TWO_LAUNCHES;
+        switch (w.kind) {
+        case KIND_Q8_0: rc = launch_kind<Q8>(w, nullptr, xq, xs, y, s, x); break;
+        case KIND_Q4_K: rc = launch_kind<Q4K>(w, nullptr, xq, xs, y, s, x); break;
+        case KIND_Q3_K:
+            rc = w.sb_lb ? launch_sb<Q3KSB>(w, nullptr, xq, xs, y, s, x) : launch_kind<Q3K>(w, nullptr, xq, xs, y, s, x);
+            break;
+        }
+        if (rc != TWO_LAUNCHES) return rc;
+    }
+    launch_quant_act(x, w.n, xq, xs, s);
+    return launch_matvec(w, nullptr, xq, xs, y, s);
 }
 
 int launch_block_dots(const Weight& w, const int8_t* xq, int32_t* dots, hipStream_t s) {

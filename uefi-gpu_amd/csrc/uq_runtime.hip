@@ -457,9 +457,7 @@ int uq_matvec_static(uq_weight_t w, const float* x, float* y, void* stream) {
     const hipStream_t s = pick(stream);
     // every code and scale the matvec reads is written by this quantization
     // first, so the scratch needs no clearing
-    launch_quant_act(x, W.n, xq, xs, s);
-    UQ_CHECK_HIP(hipGetLastError());
-    if (int rc = launch_matvec(W, nullptr, xq, xs, y, s)) return rc;
+    if (int rc = launch_matvec_x(W, x, y, xq, xs, s)) return rc;
     UQ_CHECK_HIP(hipGetLastError());
     return OK;
 }

@@ -90,7 +90,11 @@ constexpr int GBM = 32;                    // rows per workgroup tile
 // f32 rescale), so occupancy hides more than ring depth there: 2 stages fit
 // four gate/up workgroups per CU where 4 stages fit two (gate+up 104 -> 76 us
 // at 512 tokens; 3 stages changed nothing). The narrow launches wait on
-// their stage loads at 3 waves per SIMD and fill 4 stages, two at a time.
+// their stage loads at 3 waves per SIMD and fill 4 stages, two at a time; with
+// one or two workgroups per CU, 8 stages, of which 4 to 6 are in flight. A SIMD
+// then runs one or two waves, each bound by its own instruction stream, so the
+// full stages go in passes of 4 that know their ring slot and that every stage
+// they request is a full one: 134 -> 79 instructions per stage.
 
 // WM = MFMA row tiles per wave: WM 2 gives waves of 32 rows x 16 tokens
 // (workgroup 32 x 64), WM 1 waves of 16 rows x 16 tokens in a 2 x 2 grid
@@ -425,12 +429,9 @@ __device__ __forceinline__ void rope_store(const PfRopeEpi& e, int64_t t, int r,
     }
 }
 
-template <bool GU, int WM>
+// RG: the ring's stages, a power of two.
+template <bool GU, int WM, int RG>
 __global__ __launch_bounds__(256) void k_pf_gemm(PfGemmArgs a) {
-    // ring stages: the gate/up pair and the wide tiles fill two, one ahead
-    // (four would halve their workgroups per CU); the narrow launches (WM 1)
-    // fill four, two at a time, with one wait and barrier per pair of stages
-    constexpr int RG = GU || WM == 2 ? 2 : 4;
     __shared__ __attribute__((aligned(16))) GemmStageLds<GU, WM> ring[RG];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -459,43 +460,67 @@ __global__ __launch_bounds__(256) void k_pf_gemm(PfGemmArgs a) {
             gemm_issue<GU, WM>(a, src, S, r0, t0, (int64_t)s * GK_BLK, nblk_of(s), wave, lane);
         }
     };
+    auto compute_full = [&](const GemmStageLds<GU, WM>& S) {
+        // the pair block by block, the others as one group of 4
+        if constexpr (GU) {
+#pragma unroll
+            for (int j = 0; j < GK_BLK; j++) gemm_blocks<GU, WM, 1>(S, j, wc, rb, lane, f, g);
+        } else {
+            gemm_blocks<GU, WM, GK_BLK>(S, 0, wc, rb, lane, f, g);
+        }
+    };
     auto compute = [&](int s) {
         const GemmStageLds<GU, WM>& S = ring[s & (RG - 1)];
         if (s < nfull) {
-            if constexpr (GU) {
-#pragma unroll
-                for (int j = 0; j < GK_BLK; j++) gemm_blocks<GU, WM, 1>(S, j, wc, rb, lane, f, g);
-            } else {
-                gemm_blocks<GU, WM, GK_BLK>(S, 0, wc, rb, lane, f, g);
-            }
+            compute_full(S);
         } else {
             const int nblk = nblk_of(s);
             for (int j = 0; j < nblk; j++) gemm_block_tail<GU, WM>(S, j, wc, rb, lane, f, g);
         }
     };
-    // Each step: this wave's loads of the step's stages landed (nothing later
-    // is in flight), then the barrier makes every wave's loads visible and
-    // frees the ring slots the next loads fill. Full steps run in a loop with
-    // no other path, so the accumulators stay in their registers.
-    constexpr int STEP = RG / 2;
-    for (int s = 0; s < STEP && s < nst; s++) issue(s);
+    // Each step: this wave's loads of the step's stages landed (those of the
+    // RG - 2 STEP stages after them may be in flight), then the barrier makes
+    // every wave's loads visible and frees the ring slots the next loads fill.
+    // Full steps run in a loop with no other path, so the accumulators stay in
+    // their registers.
+    constexpr int STEP = RG > 2 ? 2 : 1, AHEAD = RG - 2 * STEP;
+    constexpr int LOADS = (GU ? 2 : 1) + WM, SCL = GemmStageLds<GU, WM>::SC_LOADS;  // a wave's loads per stage
+    auto wait_step = [&](int s) {
+        if (AHEAD == 0 || s + STEP + AHEAD > nst) wait_vm<0>();
+        else if (wave < SCL) wait_vm<AHEAD * (LOADS + 1)>();
+        else wait_vm<AHEAD * LOADS>();
+    };
+    for (int s = 0; s < RG - STEP && s < nst; s++) issue(s);
     int s = 0;
-    for (; s + STEP <= nfull; s += STEP) {
-        wait_vm<0>();
-        stage_barrier();
+    // UN stages per pass, every stage they load a full one
+    if constexpr (!GU && WM == 1) {
+        constexpr int UN = 4;
+        for (; s + UN + RG - STEP <= nfull; s += UN) {
+            const int h = RG == UN ? 0 : s & (RG - 1);
 #pragma unroll
-        for (int u = STEP; u < 2 * STEP; u++)
-            if (s + u < nst) issue(s + u);
+            for (int p = 0; p < UN; p += STEP) {
+                if (wave < SCL) wait_vm<AHEAD * (LOADS + 1)>();
+                else wait_vm<AHEAD * LOADS>();
+                stage_barrier();
 #pragma unroll
-        for (int u = 0; u < STEP; u++) {
-            // the pair block by block, the others as one group of 4
-            if constexpr (GU) {
+                for (int u = 0; u < STEP; u++) {
+                    gemm_issue_full<GU, WM>(cur, src, ring[(h + p + RG - STEP + u) & (RG - 1)], wave, lane);
+                    cur.advance(a.n);
+                    src.so += src.sstep;
+                }
 #pragma unroll
-                for (int j = 0; j < GK_BLK; j++) gemm_blocks<GU, WM, 1>(ring[(s + u) & (RG - 1)], j, wc, rb, lane, f, g);
-            } else {
-                gemm_blocks<GU, WM, GK_BLK>(ring[(s + u) & (RG - 1)], 0, wc, rb, lane, f, g);
+                for (int u = 0; u < STEP; u++) compute_full(ring[h + p + u]);
             }
         }
+    }
+    for (; s + STEP <= nfull; s += STEP) {
+        wait_step(s);
+        stage_barrier();
+#pragma unroll
+        for (int u = RG - STEP; u < RG; u++)
+            if (s + u < nst) issue(s + u);
+#pragma unroll
+        for (int u = 0; u < STEP; u++) compute_full(ring[(s + u) & (RG - 1)]);
     }
     if (s < nst) {
         // fewer than STEP full stages and / or the partial stage remain, all issued
@@ -851,16 +876,25 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t s) {
     // workgroups per CU; then 32 x 32 tiles of 16 x 16 waves
     if (a.yq && (!a.w2_qs || !a.yst)) return -1;
     // the quantizing gate/up epilogue needs a wave's tile to hold whole blocks (wide tiles)
-    const bool narrow = !a.yq && (a.n / GBM) * (a.mp / 64) < 4 * (int64_t)cu_count();
-    if (narrow) {
-        const dim3 grid((unsigned)(a.n / GBM), (unsigned)(a.mp / gemm_bn<1>()));
-        if (a.w2_qs) hipLaunchKernelGGL((k_pf_gemm<true, 1>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_pf_gemm<false, 1>), grid, dim3(256), 0, s, a);
+    const int64_t cu = cu_count();
+    const bool narrow = !a.yq && (a.n / GBM) * (a.mp / 64) < 4 * cu;
+    const dim3 grid((unsigned)(a.n / GBM), (unsigned)(a.mp / (narrow ? gemm_bn<1>() : gemm_bn<2>())));
+    const int64_t wgs = (int64_t)grid.x * grid.y;
+#define UQ_GEMM(GU, WM, RG) hipLaunchKernelGGL((k_pf_gemm<GU, WM, RG>), grid, dim3(256), 0, s, a)
+    if (a.w2_qs) {
+        if (narrow) UQ_GEMM(true, 1, 2);
+        else UQ_GEMM(true, 2, 2);
+    } else if (narrow) {
+        // A ring of 8 stages leaves room for two workgroups per CU. Measured in
+        // a layer at K = 8960: 96 workgroups 26.7 -> 18.1 us, 384 26.2 -> 23.7,
+        // 768 31.0 -> 39.4; at K = 1536: 96 6.3 -> 5.4 us, 128 7.4 -> 6.4, 256
+        // 7.5 -> 6.8, 512 8.2 -> 8.7 (12 stages are too few to pay for the fill).
+        if (wgs <= (a.k >= 4096 ? 2 : 1) * cu) UQ_GEMM(false, 1, 8);
+        else UQ_GEMM(false, 1, 4);
     } else {
-        const dim3 grid((unsigned)(a.n / GBM), (unsigned)(a.mp / gemm_bn<2>()));
-        if (a.w2_qs) hipLaunchKernelGGL((k_pf_gemm<true, 2>), grid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_pf_gemm<false, 2>), grid, dim3(256), 0, s, a);
+        UQ_GEMM(false, 2, 2);
     }
+#undef UQ_GEMM
     return 0;
 }
 void launch_gather_rows(const int8_t* src, int64_t rowb, const int* perm, int64_t m, int8_t* dst, hipStream_t s) {

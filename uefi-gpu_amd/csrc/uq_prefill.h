@@ -71,6 +71,7 @@ struct PfAttnArgs {
     float* xst;
     int mp;
     int ncu;                 // set by the launcher: the CU count (workgroup pairing order)
+    int sst;                 // set by the launcher: floats from one query's scores to the next in LDS
 };
 
 void launch_transpose_scales(const uint16_t* d, int64_t rows, int64_t nb, float* dt, hipStream_t s);

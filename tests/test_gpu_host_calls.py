@@ -30,6 +30,25 @@ def test_batch_output_sizes(gpu, ms):
         assert np.array_equal(y.view(np.uint32), O.matvec(O.Q8_0, r, n, m, x).view(np.uint32))
 
 
+def test_batch_after_a_refused_batch(gpu):
+    """A group that holds a kind the int8 linears do not take is refused before
+    anything is launched, so that nothing it started stores into the pinned buffer
+    of the next call, whose longer x lies where its outputs would have been."""
+    short, m = 256, 600  # 1800 outputs: stored to pinned memory by the kernels
+    refused = [uq.Weight(k, short, m, uq.synth_quant(k, 5, m, short))
+               for k in (uq.KIND_Q8_0, uq.KIND_Q4_K, uq.KIND_IQ4_XS)]
+    n = 1536
+    raws = [uq.synth_quant(uq.KIND_Q8_0, 9 + i, 600, n) for i in range(3)]
+    ws = [uq.Weight(uq.KIND_Q8_0, n, 600, r) for r in raws]
+    for seed in range(4):
+        with pytest.raises(uq.UqError) as e:
+            uq.batch(refused, uq.synth_normal(seed, short))
+        assert e.value.status == uq.Error.QUANT_TYPE
+        x = uq.synth_normal(100 + seed, n)
+        for r, y in zip(raws, uq.batch(ws, x)):
+            assert np.array_equal(y.view(np.uint32), O.matvec(O.Q8_0, r, n, 600, x).view(np.uint32))
+
+
 @pytest.mark.parametrize("m", [2048, 2049, 100000])
 def test_linear_output_sizes(gpu, m):
     n = 256

@@ -510,9 +510,14 @@ int uq_batch(const uq_weight_t* ws, int count, const float* x, int64_t n, float*
         if (int rc = ensure_y((size_t)total)) return rc;
     float* const dy = direct ? hy : g_ctx.dy;
     hipStream_t s = g_ctx.stream;
+    for (int i = 0; i < count; i++) {
+        const uint32_t k = ws[i]->w.kind;
+        if (k != KIND_Q8_0 && k != KIND_Q4_K && k != KIND_Q3_K) return set_error(ERR_QUANT_TYPE, "matvec: unsupported kind");
+    }
     launch_quant_act(hx, n, g_ctx.dxq, g_ctx.dxs, s);
     int64_t off = 0;
     bool q8 = true;
+    int rc = OK;
     for (int i = 0; i < count; i++) q8 = q8 && ws[i]->w.kind == KIND_Q8_0;
     if (q8 && count > 1) {
         // one launch for the batch (the reference's QKV job batch)
@@ -523,16 +528,21 @@ int uq_batch(const uq_weight_t* ws, int count, const float* x, int64_t n, float*
             yl[i] = dy + off;
             off += ms[i];
         }
-        if (int rc = launch_matvec_multi(wl, nullptr, yl, count, g_ctx.dxq, g_ctx.dxs, s)) return rc;
+        rc = launch_matvec_multi(wl, nullptr, yl, count, g_ctx.dxq, g_ctx.dxs, s);
     } else {
-        for (int i = 0; i < count; i++) {
-            if (int rc = launch_matvec(ws[i]->w, nullptr, g_ctx.dxq, g_ctx.dxs, dy + off, s)) return rc;
+        for (int i = 0; i < count && rc == OK; i++) {
+            rc = launch_matvec(ws[i]->w, nullptr, g_ctx.dxq, g_ctx.dxs, dy + off, s);
             off += ms[i];
         }
     }
-    if (!direct) launch_copy(hy, dy, sizeof(float) * (size_t)total, s);
-    UQ_CHECK_HIP(hipGetLastError());
-    UQ_CHECK_HIP(wait_host());
+    if (rc == OK && !direct) launch_copy(hy, dy, sizeof(float) * (size_t)total, s);
+    hipError_t e = hipGetLastError();
+    // what a failed call did launch still reads and writes the pinned buffer,
+    // which the next call fills from the host
+    const hipError_t es = wait_host();
+    if (e == hipSuccess) e = es;
+    if (rc != OK) return rc;
+    if (e != hipSuccess) return set_error(ERR_DEVICE, std::string("batch: ") + hipGetErrorString(e));
     off = 0;
     bool finite = true;
     for (int i = 0; i < count; i++) {

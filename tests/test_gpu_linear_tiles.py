@@ -102,3 +102,25 @@ def test_job_table_forms_equal_single_calls(gpu, sizes):
         pairs.append((uq.Weight(kind, n, m, uq.synth_quant(kind, i, m, n)), uq.synth_normal(i, n)))
     for (w, x), y in zip(pairs, uq.linear_batch(pairs)):
         assert np.array_equal(y.view(np.uint32), uq.linear(w, x).view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", [uq.KIND_Q8_0, uq.KIND_Q6_K])
+def test_negative_values_far_below_their_group(gpu, kind):
+    """Values that lie more than 2^62 below the largest of their 256 are no whole
+    number of the group's unit, whatever their sign. The largest meets a zero code,
+    so that only the small ones are in the sum."""
+    n, m = 512, 33
+    raw = uq.synth_quant(kind, 0x2E6 + kind, m, n).reshape(m, -1)
+    if kind == uq.KIND_Q8_0:
+        raw[:, 2] = 0
+    else:  # code 32: low bits 0, high bits 2
+        raw[:, 0] &= 0xF0
+        raw[:, 128] = (raw[:, 128] & 0xFC) | 2
+    raw = raw.reshape(-1)
+    rng = np.random.default_rng(kind)
+    for lo, hi in ((-36, -30), (-24, -21), (-19, -17), (-15, -12)):
+        x = np.zeros(n, np.float32)
+        x[1:256] = -(10.0 ** rng.uniform(lo, hi, 255))
+        x[0] = 1.0
+        y = uq.linear(uq.Weight(kind, n, m, raw), x)
+        assert ulps(y, O.linear(kind, raw, n, m, x)).max() <= 1, (lo, hi)

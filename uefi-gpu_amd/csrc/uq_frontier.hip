@@ -432,16 +432,16 @@ __device__ __forceinline__ uint64_t stage_x(const float* __restrict__ x, int n, 
                             4 * q < n ? v4.w : 0.0f};
         const float amax = uq_group_max<64>(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
         int E = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 255);
+        bool ok = E < 255;  // (a NaN is not its own floor below)
         E = E < 1 ? 1 : (E > 254 ? 254 : E);
         const double up = __builtin_bit_cast(double, (uint64_t)(188 - E + 1023) << 52);
-        bool ok = true;
         uint32_t lo[4], hi[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            // X = x * 2^(188 - E) as 2^32 * h + l, 0 <= l < 2^32: both exact, and X
-            // is whole where l has no fraction (not so for infinities and NaN)
+            // X = x * 2^(188 - E) as 2^32 * h + l, 0 <= l < 2^32: exact where X is
+            // whole. (l alone does not show it: just below zero it rounds to 2^32.)
             const double X = (double)v[k] * up, h = __builtin_floor(X * 0x1p-32), l = __builtin_fma(h, -0x1p32, X);
-            ok = ok && l == __builtin_floor(l);
+            ok = ok && X == __builtin_floor(X);
             // offset binary: digit d = byte d of (X + 0x8080808080808080) - 0x80
             const uint64_t Y = ((uint64_t)(uint32_t)(int)h << 32 | (uint32_t)l) + 0x8080808080808080ull;
             lo[k] = (uint32_t)Y ^ 0x80808080u;

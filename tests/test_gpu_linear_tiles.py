@@ -124,3 +124,51 @@ def test_negative_values_far_below_their_group(gpu, kind):
         x[0] = 1.0
         y = uq.linear(uq.Weight(kind, n, m, raw), x)
         assert ulps(y, O.linear(kind, raw, n, m, x)).max() <= 1, (lo, hi)
+
+
+SCALE_AT = {uq.KIND_Q8_0: 0, uq.KIND_IQ4_NL: 0, uq.KIND_IQ4_XS: 0, uq.KIND_IQ3_XXS: 0, uq.KIND_Q6_K: 208}
+
+
+def linear_dev(kind, n, m, raw, x):
+    """uq_linear_dev, which gives non-finite outputs where uq_linear refuses."""
+    w = uq.Weight(kind, n, m, raw)
+    L = uq.lib()
+    dx, dy = ctypes.c_void_p(), ctypes.c_void_p()
+    assert L.uq_dev_alloc(4 * n, ctypes.byref(dx)) == 0 and L.uq_dev_alloc(4 * m, ctypes.byref(dy)) == 0
+    try:
+        assert L.uq_memcpy_h2d(dx, x.ctypes.data, 4 * n) == 0
+        assert L.uq_linear_dev(w.handle, dx, dy, None) == 0
+        y = np.empty(m, np.float32)
+        assert L.uq_memcpy_d2h(y.ctypes.data, dy, 4 * m) == 0
+    finally:
+        L.uq_dev_free(dx)
+        L.uq_dev_free(dy)
+    return y
+
+
+def test_rows_beside_an_infinite_scale_keep_their_bits(gpu):
+    """A row that is not finite is summed again, in another order; the other rows of
+    its tile stay as they are. They hold pairs that cancel and a rest some 2^-44 of
+    them, so that a sum of products in double differs in the leading bits, while
+    the integer digits give the rest exactly."""
+    n, m = 544, 40
+    rng = np.random.default_rng(3)
+    codes = np.zeros((m, n), np.int8)
+    codes[:, :256] = rng.integers(-127, 128, (m, 256))
+    codes[:, 256:512] = -codes[:, :256]
+    codes[:, 512:] = rng.integers(-127, 128, (m, 32))
+    raw = np.zeros((m, n // 32, 34), np.uint8)
+    raw[:, :, 1] = 0x3C  # every scale 1.0
+    raw[:, :, 2:] = codes.view(np.uint8).reshape(m, n // 32, 32)
+    x = np.zeros(n, np.float32)
+    x[:256] = rng.normal(0, 1, 256) * 2.0 ** rng.integers(-24, 1, 256)
+    x[256:512] = x[:256]
+    x[512:] = rng.normal(0, 1, 32) * 2.0 ** -44
+    exact = (codes[:, 512:].astype(np.float64) * x[512:].astype(np.float64)).sum(1).astype(np.float32)
+    clean = linear_dev(uq.KIND_Q8_0, n, m, raw.reshape(-1), x)
+    assert ulps(clean, exact).max() <= 1
+    raw[20, 3, 1] = 0x7C
+    y = linear_dev(uq.KIND_Q8_0, n, m, raw.reshape(-1), x)
+    assert not np.isfinite(y[20])
+    rest = np.arange(m) != 20
+    assert np.array_equal(y[rest].view(np.uint32), clean[rest].view(np.uint32))

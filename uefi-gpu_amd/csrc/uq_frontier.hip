@@ -908,7 +908,7 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
     const XStage xs = stage();
     // Tiles [from, to) of the workgroup: one wave sums a tile's segments, then
     // its four lane groups.
-    bool nan = false;
+    bool again = false;
     auto sum_tiles = [&](int from, int to, int buffer, uint64_t mask) {
         __syncthreads();
         for (int i = from + wave; i < to; i += FL_SEGS) {
@@ -922,8 +922,9 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
             const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
             if (mask) top += wide_products<T>(j, tile, S, mask, ln, xs);
             const double sum = uq_swap32_sum(uq_swap16_sum(top));
-            nan = nan || sum != sum;
-            if (ln.g == 0 && row < j.m) j.y[row] = (float)sum;
+            const bool finite = __builtin_fabs(sum) < __builtin_inf();
+            again = again || !finite;
+            if (ln.g == 0 && row < j.m) j.y[row] = finite ? (float)sum : __builtin_nanf("");
         }
     };
     auto combine = [&](const double (&acc)[4]) {
@@ -966,16 +967,18 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         }
 #pragma unroll 1
         while (base < count) flush();
-        // A zero digit times an infinite scale is NaN where the row's own
-        // products are not: the tiles of a wave that saw one run again, wholly
-        // in double.
-        if (__builtin_amdgcn_ballot_w64(nan) == 0) return;
+        // A zero digit times an infinite scale is NaN where the row's own products
+        // are not: the rows that came out so, and only they, run again wholly in
+        // double.
+        if (__builtin_amdgcn_ballot_w64(again) == 0) return;
 #pragma unroll 1
         for (int i = 0; i < count; i++) {
             if (((i % dep) & (FL_SEGS - 1)) != wave) continue;
             const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
+            const bool redo = ln.g == 0 && row < j.m && j.y[row] != j.y[row];  // the lane's own stores
+            if (__builtin_amdgcn_ballot_w64(redo) == 0) continue;
             const double sum = uq_swap32_sum(uq_swap16_sum(wide_products<T>(j, tile, S, ~0ull, ln, xs)));
-            if (ln.g == 0 && row < j.m) j.y[row] = (float)sum;
+            if (redo) j.y[row] = (float)sum;
         }
         return;
     }

@@ -172,3 +172,32 @@ def test_rows_beside_an_infinite_scale_keep_their_bits(gpu):
     assert not np.isfinite(y[20])
     rest = np.arange(m) != 20
     assert np.array_equal(y[rest].view(np.uint32), clean[rest].view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("signs", ["one", "both"])
+def test_infinite_scale_gives_what_the_products_give(gpu, kind, wide, signs):
+    """A row with an infinite scale is an infinity where its products have one sign
+    and NaN where they have both (or a zero code), with and without groups of x that
+    run in double."""
+    n, m, row = 1024, 40, 20
+    raw = uq.synth_quant(kind, 0x41F + kind, m, n)
+    rb = uq.row_bytes(kind, n)
+    if kind == uq.KIND_Q8_0:
+        codes = raw[row * rb:(row + 1) * rb].reshape(-1, 34)[:, 2:]
+        codes[codes == 0] = 1
+    weights = O.dequantize(kind, raw[row * rb:(row + 1) * rb], n)
+    x = np.abs(uq.synth_normal(kind + 9, n)) * np.where(weights < 0, np.float32(-1), np.float32(1))
+    if signs == "both":
+        x[1] = -x[1]
+    if wide:
+        x[[2, 600]] = 1e-20 * np.sign(x[[2, 600]])
+    raw[row * rb + SCALE_AT[kind]], raw[row * rb + SCALE_AT[kind] + 1] = 0x00, 0x7C
+    y = linear_dev(kind, n, m, raw, x)
+    ref = O.linear(kind, raw, n, m, x)
+    rest = np.arange(m) != row
+    assert ulps(y[rest], ref[rest]).max() <= 1
+    assert (np.isnan(y[row]) and np.isnan(ref[row])) or y[row] == ref[row]
+    if signs == "one" and kind in (uq.KIND_Q8_0, uq.KIND_IQ4_NL, uq.KIND_IQ3_XXS):
+        assert y[row] == np.inf  # (no zero code or sub-scale in these)

@@ -828,17 +828,19 @@ __device__ double wide_products(const FJob& j, int64_t tile, int S, uint64_t mas
             uint32_t c[4];
             int col = 0;
             const double s = T::chunk(u, ln, t, k, c, &col);
-            double d[4] = {0.0, 0.0, 0.0, 0.0};
             if (col < xs.n) {
+                // weight by weight: the products of an infinite scale have signs of
+                // their own, which the sum of a chunk would hide
+                double d[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const float4 x4 = *(const float4*)(xs.xg + col + 4 * q);
                     const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        d[i] = __builtin_fma((double)(int)(int8_t)(uint8_t)(c[q] >> (8 * i)), (double)xv[i], d[i]);
+                        d[i] = __builtin_fma(s * (double)(int)(int8_t)(uint8_t)(c[q] >> (8 * i)), (double)xv[i], d[i]);
                 }
-                r = __builtin_fma(s, (d[0] + d[1]) + (d[2] + d[3]), r);
+                r += (d[0] + d[1]) + (d[2] + d[3]);
             }
         }
     }
@@ -927,6 +929,20 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
             if (ln.g == 0 && row < j.m) j.y[row] = finite ? (float)sum : __builtin_nanf("");
         }
     };
+    // A zero digit times an infinite scale is NaN where the row's own products are
+    // not: the rows that came out so, and only they, run again wholly in double.
+    auto sum_again = [&]() {
+        if (__builtin_amdgcn_ballot_w64(again) == 0) return;
+#pragma unroll 1
+        for (int i = 0; i < count; i++) {
+            if (xs.wide ? wave != 0 : ((i % dep) & (FL_SEGS - 1)) != wave) continue;
+            const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
+            const bool redo = ln.g == 0 && row < j.m && j.y[row] != j.y[row];  // the lane's own stores
+            if (__builtin_amdgcn_ballot_w64(redo) == 0) continue;
+            const double sum = uq_swap32_sum(uq_swap16_sum(wide_products<T>(j, tile, S, ~0ull, ln, xs)));
+            if (redo) j.y[row] = (float)sum;
+        }
+    };
     auto combine = [&](const double (&acc)[4]) {
         double t = __builtin_fma(acc[3], 256.0, acc[2]);
         t = __builtin_fma(t, 256.0, acc[1]);
@@ -967,19 +983,7 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         }
 #pragma unroll 1
         while (base < count) flush();
-        // A zero digit times an infinite scale is NaN where the row's own products
-        // are not: the rows that came out so, and only they, run again wholly in
-        // double.
-        if (__builtin_amdgcn_ballot_w64(again) == 0) return;
-#pragma unroll 1
-        for (int i = 0; i < count; i++) {
-            if (((i % dep) & (FL_SEGS - 1)) != wave) continue;
-            const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
-            const bool redo = ln.g == 0 && row < j.m && j.y[row] != j.y[row];  // the lane's own stores
-            if (__builtin_amdgcn_ballot_w64(redo) == 0) continue;
-            const double sum = uq_swap32_sum(uq_swap16_sum(wide_products<T>(j, tile, S, ~0ull, ln, xs)));
-            if (redo) j.y[row] = (float)sum;
-        }
+        sum_again();
         return;
     }
     // Some group of x is wide: without the ring, tile by tile.
@@ -997,6 +1001,7 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         }
         sum_tiles(i, i + 1, i & 1, xs.wide);
     }
+    sum_again();
 }
 
 // ---- F32 / BF16 rows

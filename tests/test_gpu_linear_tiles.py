@@ -201,3 +201,73 @@ def test_infinite_scale_gives_what_the_products_give(gpu, kind, wide, signs):
     assert (np.isnan(y[row]) and np.isnan(ref[row])) or y[row] == ref[row]
     if signs == "one" and kind in (uq.KIND_Q8_0, uq.KIND_IQ4_NL, uq.KIND_IQ3_XXS):
         assert y[row] == np.inf  # (no zero code or sub-scale in these)
+
+
+def far_x(n, seed, share):
+    """Ordinary values, `share` of each group of 256 more than 2^38 below its largest
+    (some denormal, some zero)."""
+    rng = np.random.default_rng(seed)
+    x = rng.normal(0, 1, n).astype(np.float32)
+    far = rng.random(n) < share
+    far[5::256] = True
+    x[far] *= np.float32(2.0) ** rng.integers(-140, -40, far.sum())
+    return x
+
+
+def repeated_rows(kind, n, m, seed, rows=997):
+    """Rows 0 .. 996 over and over: a weight of m rows and the raw bytes of the 997."""
+    raw = uq.synth_quant(kind, seed, rows, n)
+    return raw, np.resize(raw.reshape(rows, -1), (m, raw.size // rows)).reshape(-1)
+
+
+def check_repeated(y, ref, m):
+    assert ulps(y[:ref.size], ref).max() <= 1
+    assert np.array_equal(y.view(np.uint32), np.resize(y[:ref.size], m).view(np.uint32))
+
+
+# n 2048: more than eight tiles a workgroup, four of them summed at once, and the
+# buffers used again; 512: fewer steps than waves; 8192: x leaves room for one
+# tile's sums at once
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("n,m", [(2048, 150001), (512, 150001), (8192, 30011)])
+@pytest.mark.parametrize("share", [None, 0.004, 0.5])
+def test_sums_of_many_tiles(gpu, kind, n, m, share):
+    x = uq.synth_normal(n, n) if share is None else far_x(n, n, share)
+    raw, big = repeated_rows(kind, n, m, 0x6B1 + kind)
+    y = uq.linear(uq.Weight(kind, n, m, big), x)
+    check_repeated(y, O.linear(kind, raw, n, 997, x), m)
+
+
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("wide", [False, True])
+def test_infinite_scales_in_late_tiles(gpu, kind, wide):
+    """Every wave finds its own rows again: infinite scales in tiles all over a
+    workgroup's."""
+    n, m = 1024, 60011
+    raw, big = repeated_rows(kind, n, m, 0x6C1 + kind)
+    rb = uq.row_bytes(kind, n)
+    bad = np.arange(7, m, 1999)
+    at = bad * rb + SCALE_AT[kind]
+    big[at], big[at + 1] = 0x00, 0x7C
+    x = far_x(n, n, 0.01) if wide else uq.synth_normal(n, n)
+    y = linear_dev(kind, n, m, big, x)
+    assert not np.isfinite(y[bad]).any()
+    for r in bad[:: max(1, len(bad) // 8)]:
+        ref = O.linear(kind, big[r * rb:(r + 1) * rb], n, 1, x)[0]
+        assert (np.isnan(y[r]) and np.isnan(ref)) or y[r] == ref
+    ref = O.linear(kind, raw, n, 997, x)
+    good = np.setdiff1d(np.arange(m), bad)
+    assert ulps(y[good], np.resize(ref, m)[good]).max() <= 1
+
+
+def test_far_values_in_a_job_table(gpu):
+    """A table in which some jobs' x have such values gives the bits of the single
+    calls."""
+    pairs = []
+    for i, m in enumerate([700, 33, 5000, 16, 1, 900, 64]):
+        kind = TILE_KINDS[i % len(TILE_KINDS)]
+        n = (512, 2560)[i % 2]
+        x = far_x(n, i, 0.02) if i % 3 else uq.synth_normal(i, n)
+        pairs.append((uq.Weight(kind, n, m, uq.synth_quant(kind, i, m, n)), x))
+    for (w, x), y in zip(pairs, uq.linear_batch(pairs)):
+        assert np.array_equal(y.view(np.uint32), uq.linear(w, x).view(np.uint32))

@@ -368,9 +368,10 @@ struct FJob {
 // x is staged in LDS as integers X_j with x_j = X_j * 2^(E - 188) in groups of
 // 256 values: E = max(biased exponent of max|x_j|, 1), |X_j| < 2^62, exact when
 // every element lies within 2^38 of the group's maximum (or has zeros in the
-// bits that fall away). X_j is held as eight balanced base-256 digits. A group that is
-// not exact (wider range, or a non-finite value) has digits 0 and a bit in
-// `wide`; its products run in double from x itself.
+// bits that fall away). X_j is held as eight balanced base-256 digits. Four values
+// with one among them that is not exact (wider range, or not finite) have digits 0
+// and a bit in their group's `far`, the group one in `wide`; their products run in
+// double from x itself.
 //
 // The dots run on v_mfma_i32_16x16x64_i8 with the weights of 16 rows as one
 // operand and the digits as the other, so one instruction forms all eight
@@ -388,9 +389,10 @@ constexpr int XDIG = 8, XGROUP = 256, XCHUNK = 16 * (XDIG + 1);
 struct XStage {
     const uint8_t* dig;
     const double* gexp;   // per group: 2^(E - 188)
-    const float* xg;      // x in global memory (wide groups)
+    const uint64_t* far;  // per group: bit q: values 4q .. 4q + 3 run in double
+    const float* xg;      // x in global memory (those values)
     const float* xf;      // F32 / BF16 weights: x as f32 in LDS
-    uint64_t wide;        // bit g: group g runs in double
+    uint64_t wide;        // bit g: group g has such values
     int n;
 };
 
@@ -422,7 +424,7 @@ __device__ __forceinline__ void load_ahead(const float* __restrict__ x, int n, f
 // Stages x of one job, one 256-value group per wave at a time, 4 values per
 // lane; returns the wave's wide groups.
 __device__ __forceinline__ uint64_t stage_x(const float* __restrict__ x, int n, const float4 (&ahead)[XAHEAD], uint8_t* dig,
-                                            double* gexp) {
+                                            double* gexp, uint64_t* far) {
     const int lane = threadIdx.x & 63, nw = (int)blockDim.x >> 6, ng = (n + XGROUP - 1) / XGROUP;
     uint64_t wide = 0;
     const int first = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -457,10 +459,12 @@ __device__ __forceinline__ uint64_t stage_x(const float* __restrict__ x, int n, 
 #pragma unroll
             for (int k = 0; k < 4; k++) d[4 + k] = t[k];
         }
-        if (__builtin_amdgcn_ballot_w64(!ok)) {
+        const uint64_t out = __builtin_amdgcn_ballot_w64(!ok);
+        if (out) {
             wide |= 1ull << grp;
+            if (lane == 0) far[grp] = out;
 #pragma unroll
-            for (int k = 0; k < XDIG; k++) d[k] = 0;
+            for (int k = 0; k < XDIG; k++) d[k] = ok ? d[k] : 0;
         }
         const int c = q >> 2;
 #pragma unroll
@@ -639,12 +643,11 @@ struct TK<KIND_Q8_0> {
             for (int i = 0; i < 4; i++) acc[i] = __builtin_fma((double)d[p][i], s, acc[i]);
         }
     }
-    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
+    static __device__ __forceinline__ int column(const Lane& ln, int t, int k) { return VPS * t + 64 * k + 16 * ln.g; }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int k, uint32_t (&c)[4]) {
         uint32_t sc[2];
         to_slices(u.d, sc);
-        const uint4& w = k ? u.b : u.a;
-        c[0] = w.x, c[1] = w.y, c[2] = w.z, c[3] = w.w;
-        *col = VPS * t + 64 * k + 16 * ln.g;
+        c[0] = k ? u.b.x : u.a.x, c[1] = k ? u.b.y : u.a.y, c[2] = k ? u.b.z : u.a.z, c[3] = k ? u.b.w : u.a.w;
         return (double)uq_half((uint16_t)sc[k]);
     }
 };
@@ -665,9 +668,9 @@ struct TK<KIND_IQ4_NL> {
     static __device__ __forceinline__ void step(const U& u, const Lane& ln, const XStage& xs, int t, double (&acc)[4]) {
         step_f16<TK>(u, ln, xs, t, acc);
     }
-    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
+    static __device__ __forceinline__ int column(const Lane& ln, int t, int k) { return VPS * t + 32 * ln.g + 16 * k; }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane&, int k, uint32_t (&c)[4]) {
         codes(u, k, c);
-        *col = VPS * t + 32 * ln.g + 16 * k;
         return (double)uq_half((uint16_t)u.d);
     }
 };
@@ -723,11 +726,14 @@ struct BookKind {
         block_sums(x, w, si, ia);
         add_step(ia, scale_d(u) * e, acc);
     }
-    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
-        const int b = k >> 1;
-        book_codes16(book(), b ? u.b : u.a, 0, c);
-        if (k & 1) book_codes16(book(), b ? u.b : u.a, 1, c);
-        *col = VPS * t + 128 * b + 32 * ln.g + 16 * (k & 1);
+    static __device__ __forceinline__ int column(const Lane& ln, int t, int k) {
+        return VPS * t + 128 * (k >> 1) + 32 * ln.g + 16 * (k & 1);
+    }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int k, uint32_t (&c)[4]) {
+        const int b = k >> 1, sh = 4 * (k & 1);
+        const uint4 w = {(b ? u.b.x : u.a.x) >> sh, (b ? u.b.y : u.a.y) >> sh, (b ? u.b.z : u.a.z) >> sh,
+                         (b ? u.b.w : u.a.w) >> sh};
+        book_codes16(book(), w, 0, c);
         // this lane's own block 4b + g: lane groups 2p, 2p + 1 stand for slices 0, 1 of pair p,
         // and the scales of slice s sit in lane groups 2s and 2s + 1
         const int own = 2 * b + (ln.g >> 1);
@@ -804,46 +810,63 @@ struct TK<KIND_Q6_K> {
         }
         add_step(ia, (double)uq_half((uint16_t)u.d) * e, acc);
     }
-    static __device__ __forceinline__ double chunk(const U& u, const Lane& ln, int t, int k, uint32_t (&c)[4], int* col) {
-        codes(u, 0, c);
-        if (k == 1) codes(u, 1, c);
-        if (k == 2) codes(u, 2, c);
-        if (k == 3) codes(u, 3, c);
-        *col = VPS * t + 128 * (ln.g >> 1) + 16 * (ln.g & 1) + 32 * k;
+    static __device__ __forceinline__ int column(const Lane& ln, int t, int k) {
+        return VPS * t + 128 * (ln.g >> 1) + 16 * (ln.g & 1) + 32 * k;
+    }
+    static __device__ __forceinline__ double chunk(const U& u, const Lane&, int k, uint32_t (&c)[4]) {
+        // (as codes(), for a k that is not known when compiling)
+        const uint32_t lv[4] = {u.l0.x, u.l0.y, u.l0.z, u.l0.w}, lw[4] = {u.l1.x, u.l1.y, u.l1.z, u.l1.w};
+        const uint32_t hv[4] = {u.h.x, u.h.y, u.h.z, u.h.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t lo = (((k & 1) ? lw[q] : lv[q]) >> (4 * (k >> 1))) & 0x0F0F0F0Fu;
+            c[q] = ((((hv[q] >> (2 * k)) & 0x03030303u) << 4 | lo) + 0x60606060u) ^ 0x80808080u;
+        }
         return (double)uq_half((uint16_t)u.d) * (double)(int8_t)(uint8_t)(u.sc >> (8 * k));
     }
 };
 
-// Products of the groups in `mask` in double, steps [0, S) of the tile in
-// order: this lane's chunks of its row.
-template <class T>
-__device__ double wide_products(const FJob& j, int64_t tile, int S, uint64_t mask, const Lane& ln, const XStage& xs) {
+// Products of step t that run in double, this lane's chunks of its row: those of
+// x's far values, or (ALL) every one.
+template <class T, bool ALL>
+__device__ __forceinline__ double step_double(const typename T::U& u, const Lane& ln, const XStage& xs, int t) {
     double r = 0.0;
 #pragma unroll 1
-    for (int t = 0; t < S; t++) {
-        if (!((mask >> (t * T::VPS / XGROUP)) & 1)) continue;
-        const typename T::U u = T::load(j, tile, t, ln.lane);
-#pragma unroll 1
-        for (int k = 0; k < T::CHUNKS; k++) {
-            uint32_t c[4];
-            int col = 0;
-            const double s = T::chunk(u, ln, t, k, c, &col);
-            if (col < xs.n) {
-                // weight by weight: the products of an infinite scale have signs of
-                // their own, which the sum of a chunk would hide
-                double d[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int k = 0; k < T::CHUNKS; k++) {
+        const int col = T::column(ln, t, k);
+        uint32_t take = col < xs.n ? 15u : 0u;
+        if (!ALL) take &= (uint32_t)(xs.far[t * T::VPS / XGROUP] >> ((col & (XGROUP - 1)) >> 2));
+        if (__builtin_amdgcn_ballot_w64(take != 0) == 0) continue;
+        uint32_t c[4];
+        const double s = T::chunk(u, ln, k, c);
+        if (take) {
+            // ALL: weight by weight, as the products of an infinite scale have signs
+            // of their own, which the sum of a chunk would hide
+            double d[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 x4 = *(const float4*)(xs.xg + col + 4 * q);
-                    const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
+            for (int q = 0; q < 4; q++) {
+                const float4 x4 = *(const float4*)(xs.xg + col + 4 * q);
+                const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        d[i] = __builtin_fma(s * (double)(int)(int8_t)(uint8_t)(c[q] >> (8 * i)), (double)xv[i], d[i]);
+                for (int i = 0; i < 4; i++) {
+                    const double code = (double)(int)(int8_t)(uint8_t)(c[q] >> (8 * i));
+                    d[i] = ALL ? __builtin_fma(s * code, (double)xv[i], d[i])
+                               : __builtin_fma(code, (take >> q) & 1 ? (double)xv[i] : 0.0, d[i]);
                 }
-                r += (d[0] + d[1]) + (d[2] + d[3]);
             }
+            const double sum = (d[0] + d[1]) + (d[2] + d[3]);
+            r = ALL ? r + sum : __builtin_fma(s, sum, r);
         }
     }
+    return r;
+}
+
+// All products of a tile in double.
+template <class T>
+__device__ double tile_double(const FJob& j, int64_t tile, int S, const Lane& ln, const XStage& xs) {
+    double r = 0.0;
+#pragma unroll 1
+    for (int t = 0; t < S; t++) r += step_double<T, true>(T::load(j, tile, t, ln.lane), ln, xs, t);
     return r;
 }
 
@@ -909,9 +932,11 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
     for (int b = 0; b < NB; b++) fetch(buf[b]);
     const XStage xs = stage();
     // Tiles [from, to) of the workgroup: one wave sums a tile's segments, then
-    // its four lane groups.
+    // its four lane groups. A zero digit times an infinite scale is NaN where the
+    // row's own products are not: rows that are not finite, and only they, are
+    // summed again wholly in double at the end, and NaN until then.
     bool again = false;
-    auto sum_tiles = [&](int from, int to, int buffer, uint64_t mask) {
+    auto sum_tiles = [&](int from, int to, int buffer) {
         __syncthreads();
         for (int i = from + wave; i < to; i += FL_SEGS) {
             double v[FL_SEGS];
@@ -920,27 +945,12 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
                 const double t = part[((buffer * dep + (i - from)) * FL_SEGS + k) * 64 + ln.lane];
                 v[k] = k < ns ? t : 0.0;
             }
-            double top = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            const double top = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
             const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
-            if (mask) top += wide_products<T>(j, tile, S, mask, ln, xs);
             const double sum = uq_swap32_sum(uq_swap16_sum(top));
             const bool finite = __builtin_fabs(sum) < __builtin_inf();
             again = again || !finite;
             if (ln.g == 0 && row < j.m) j.y[row] = finite ? (float)sum : __builtin_nanf("");
-        }
-    };
-    // A zero digit times an infinite scale is NaN where the row's own products are
-    // not: the rows that came out so, and only they, run again wholly in double.
-    auto sum_again = [&]() {
-        if (__builtin_amdgcn_ballot_w64(again) == 0) return;
-#pragma unroll 1
-        for (int i = 0; i < count; i++) {
-            if (xs.wide ? wave != 0 : ((i % dep) & (FL_SEGS - 1)) != wave) continue;
-            const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
-            const bool redo = ln.g == 0 && row < j.m && j.y[row] != j.y[row];  // the lane's own stores
-            if (__builtin_amdgcn_ballot_w64(redo) == 0) continue;
-            const double sum = uq_swap32_sum(uq_swap16_sum(wide_products<T>(j, tile, S, ~0ull, ln, xs)));
-            if (redo) j.y[row] = (float)sum;
         }
     };
     auto combine = [&](const double (&acc)[4]) {
@@ -955,7 +965,7 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         // once the wave is past them, the workgroup sums the tiles from `base` on
         auto flush = [&]() {
             const int to = base + dep < count ? base + dep : count;
-            sum_tiles(base, to, buffer, 0);
+            sum_tiles(base, to, buffer);
             base = to;
             buffer ^= 1;
         };
@@ -983,25 +993,48 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         }
 #pragma unroll 1
         while (base < count) flush();
-        sum_again();
-        return;
-    }
-    // Some group of x is wide: without the ring, tile by tile.
+    } else {
+        // x has far values: without the ring, as the loads of x would cost it the
+        // exact waits. Each wave sums its own steps' products with them, chunks
+        // without one left out. 49344 x 2560 with one such value in x / one in
+        // each group, against one wave summing all products of a group with one:
+        // Q8_0 65.6 -> 30.6 us / 254 -> 41.7, IQ3_XXS 43.6 -> 21.6 / 214 -> 33.3.
+        int base = 0, buffer = 0;
+        auto flush = [&]() {
+            const int to = base + dep < count ? base + dep : count;
+            sum_tiles(base, to, buffer);
+            base = to;
+            buffer ^= 1;
+        };
 #pragma unroll 1
-    for (int i = 0; i < count; i++) {
-        if (p.i == i) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
+        while (p.i < count) {
+            if (p.i >= base + dep) {
+                flush();
+                continue;
+            }
+            double acc[4] = {0.0, 0.0, 0.0, 0.0}, more = 0.0;
 #pragma unroll 1
             for (; p.s < p.end; p.s++) {
-                const typename T::U u = T::load(j, wgi + i * j.wgs, p.s, ln.lane);
+                const typename T::U u = T::load(j, wgi + p.i * j.wgs, p.s, ln.lane);
+                if ((xs.wide >> (p.s * T::VPS / XGROUP)) & 1) more += step_double<T, false>(u, ln, xs, p.s);
                 T::step(u, ln, xs, p.s, acc);
             }
-            part[((i & 1) * dep * FL_SEGS + p.seg) * 64 + ln.lane] = combine(acc);
+            part[((buffer * dep + (p.i - base)) * FL_SEGS + p.seg) * 64 + ln.lane] = combine(acc) + more;
             p.next();
         }
-        sum_tiles(i, i + 1, i & 1, xs.wide);
+#pragma unroll 1
+        while (base < count) flush();
     }
-    sum_again();
+    if (__builtin_amdgcn_ballot_w64(again) == 0) return;
+#pragma unroll 1
+    for (int i = 0; i < count; i++) {
+        if (((i % dep) & (FL_SEGS - 1)) != wave) continue;
+        const int64_t tile = wgi + (int64_t)i * j.wgs, row = 16 * tile + ln.row;
+        const bool redo = ln.g == 0 && row < j.m && j.y[row] != j.y[row];  // the lane's own stores
+        if (__builtin_amdgcn_ballot_w64(redo) == 0) continue;
+        const double sum = uq_swap32_sum(uq_swap16_sum(tile_double<T>(j, tile, S, ln, xs)));
+        if (redo) j.y[row] = (float)sum;
+    }
 }
 
 // ---- F32 / BF16 rows
@@ -1153,8 +1186,8 @@ __device__ __forceinline__ FJob find_job(const JobArgs& a, int* wgi) {
     *wgi = gridDim.y == 1 ? (int)blockIdx.x - j.wg0 : ((int)blockIdx.x < j.wgs ? (int)blockIdx.x : -1);
     return j;
 }
-// Dynamic LDS of a job: the digits of x padded to whole groups and the group
-// factors (F32 / BF16 weights: x as f32).
+// Dynamic LDS of a job: the digits of x padded to whole groups, the group
+// factors and the groups' far values (F32 / BF16 weights: x as f32).
 __device__ __forceinline__ XStage stage_floats(const FJob& j, uint8_t* lds) {
     XStage xs{};
     xs.xf = (const float*)lds;
@@ -1167,12 +1200,14 @@ __device__ __forceinline__ XStage stage_digits(const FJob& j, const float4 (&ahe
     const int ng = (j.n + XGROUP - 1) / XGROUP;
     uint8_t* const dig = lds;
     double* const gexp = (double*)(lds + XCHUNK * (XGROUP / 16) * ng);
-    const uint64_t wide = stage_x(j.x, j.n, ahead, dig, gexp);
+    uint64_t* const far = (uint64_t*)(gexp + ng);
+    const uint64_t wide = stage_x(j.x, j.n, ahead, dig, gexp, far);
     if ((threadIdx.x & 63) == 0) wides[threadIdx.x >> 6] = wide;
     __syncthreads();
     XStage xs{};
     xs.dig = dig;
     xs.gexp = gexp;
+    xs.far = far;
     xs.xg = j.x;
     xs.n = j.n;
     uint64_t all = 0;
@@ -1278,7 +1313,7 @@ int fl_resident(const void* kern, size_t lds) {
 size_t stage_bytes(uint32_t kind, int n) {
     if (kind == KIND_F32 || kind == KIND_BF16) return 4 * (size_t)n;
     const size_t ng = ((size_t)n + XGROUP - 1) / XGROUP;
-    return (XCHUNK * (XGROUP / 16) + 8) * ng;
+    return (XCHUNK * (XGROUP / 16) + 8 + 8) * ng;
 }
 
 // Instructions of a wave for 16 rows per column, and of the staging per column,
@@ -1292,7 +1327,7 @@ double step_cost(uint32_t kind) {
     return 0.9;
 }
 // Tiles whose segments meet at once: 32 KB of LDS, one where x takes more than
-// 64 KB (n > 7168), so that the largest x (149 KB) still fits.
+// 64 KB (n > 7168), so that the largest x (148 KB) still fits.
 constexpr int FL_DEP = 4;
 
 bool row_kind(uint32_t kind) { return kind == KIND_F32 || kind == KIND_BF16; }

@@ -271,3 +271,15 @@ def test_far_values_in_a_job_table(gpu):
         pairs.append((uq.Weight(kind, n, m, uq.synth_quant(kind, i, m, n)), x))
     for (w, x), y in zip(pairs, uq.linear_batch(pairs)):
         assert np.array_equal(y.view(np.uint32), uq.linear(w, x).view(np.uint32))
+
+
+# either side of one and two workgroups a CU, of whole shares of the tiles and a
+# workgroup on every CU, and of the longest x that leaves LDS for two (256 CUs)
+@pytest.mark.parametrize("kind", TILE_KINDS)
+@pytest.mark.parametrize("n,m", [(512, 32768), (512, 32769), (1024, 16384), (1024, 16385), (2560, 28672), (2560, 28673),
+                                 (4096, 12288), (4096, 12289), (4096, 28673), (5376, 28673), (5632, 28673)])
+def test_workgroups_of_one_weight(gpu, kind, n, m):
+    x = uq.synth_normal(n + m, n)
+    raw, big = repeated_rows(kind, n, m, 0x6D1 + kind)
+    y = uq.linear(uq.Weight(kind, n, m, big), x)
+    check_repeated(y, O.linear(kind, raw, n, 997, x), m)

@@ -1320,9 +1320,50 @@ size_t stage_bytes(uint32_t kind, int n) {
     return (XCHUNK * (XGROUP / 16) + 8 + 8) * ng;
 }
 
+// Tiles whose segments meet at once: 32 KB of LDS, one where x takes more than
+// 64 KB (n > 7168), so that the largest x (148 KB) still fits.
+constexpr int FL_DEP = 4;
+Parts plan_parts(size_t stage, size_t* lds) {
+    const int at = (int)((stage + 15) & ~(size_t)15), dep = at <= 64 * 1024 ? FL_DEP : 1;
+    *lds = (size_t)at + 2 * 8 * 64 * FL_SEGS * (size_t)dep;
+    return {dep, at};
+}
+
+// Workgroups of a single weight of a tiled kind: one or two a CU (a third never
+// paid). MI355X, HIP events, weights that rotate past the caches, us:
+//  * Where LDS holds one (n > 5376) the second only waits: 32000 x 7168 with
+//    256 / 512 workgroups Q8_0 46.4 / 49.9, Q6_K 35.4 / 38.1, IQ4_XS 32.4 / 35.1.
+//  * The IQ kinds are bound by the VALU and need four waves per SIMD once there
+//    are tiles enough: 13000 x 2560 (3.2 tiles a CU) IQ4_XS 7.3 / 7.9, 20000 9.2 /
+//    8.7, 49344 20.1 / 16.2, 151936 52.8 / 40.4; 100000 x 256 8.7 / 7.1, 70000 7.0 /
+//    6.9; 13000 x 4096 IQ4_NL 12.3 / 11.5.
+//  * Q8_0 reads at the memory's rate with two waves per SIMD and two steps in
+//    flight: 100000 x 2560 52.8 / 54.0, 151936 77.2 / 79.3, 40000 x 4096 33.8 /
+//    35.3. Short rows leave a wave one step or two per tile: 151936 x 2048 65.5 /
+//    63.5, 100000 x 1024 25.6 / 21.5, 18000 x 1536 (4.4 tiles a CU) 8.6 / 9.1.
+//  * Q6_K is between: 100000 x 2560 36.9 / 38.6, 128256 x 3072 55.5 / 52.9, 100000 x
+//    3072 45.4 / 46.9, x 1024 17.2 / 17.1, x 256 9.0 / 7.7, 49344 x 4096 30.0 / 28.6.
+// All CUs get one where there are many tiles: 49344 rows as 238 workgroups of 13
+// tiles / 256 of 12 or 13, Q8_0 29.8 / 29.0. With few tiles, and Q6_K always,
+// whole shares cost less: 13000 x 7168 as 204 of 4 / 256 of 3 or 4, Q6_K 18.0 / 19.5,
+// Q8_0 25.1 / 25.5.
+int64_t single_wgs(uint32_t kind, int64_t n, int64_t tiles, size_t lds, int64_t cu) {
+    const bool q8 = kind == KIND_Q8_0, q6 = kind == KIND_Q6_K;
+    const bool fits = 2 * lds <= 160 * 1024;
+    const int64_t from = n >= 4096 ? (q6 ? 7 : 3) : (n >= 1024 ? (q8 ? 5 : 4) : 3 + 1536 / n);  // tiles a CU
+    const bool two = fits && tiles > from * cu && (q8 ? n < 2560 : (q6 ? n < 1024 || n >= 4096 : true));
+    if (two) return std::min(tiles, 2 * cu);
+    const int64_t nt = (tiles + cu - 1) / cu;
+    return q6 || nt < 8 ? (tiles + nt - 1) / nt : cu;
+}
+
 // Instructions of a wave for 16 rows per column, and of the staging per column,
-// relative to each other.
-constexpr double STAGE_COST = 0.55;  // about 130 instructions per 256 columns against 190 for a step of them
+// in proportion to each other: the table planner's weights. Counted, not fitted;
+// what they choose was held against 1 to 20 tiles a workgroup: 22 IQ3_XXS 640 x
+// 2560 beside an F32 router 8.44 us (4 tiles; best 8.41), eight IQ4_XS 2560 x 2560
+// 9.93 (9.90), a Q8_0 q|k|v 7.61 (7.61). Tables of very unequal row lengths are
+// not at their best: 2560 x 16384 with six of 2560 x 512 (Q6_K) 39.2 (21.0 with 2).
+constexpr double STAGE_COST = 0.55;
 double step_cost(uint32_t kind) {
     switch (kind) {
     case KIND_Q8_0: return 0.5;
@@ -1330,9 +1371,6 @@ double step_cost(uint32_t kind) {
     }
     return 0.9;
 }
-// Tiles whose segments meet at once: 32 KB of LDS, one where x takes more than
-// 64 KB (n > 7168), so that the largest x (148 KB) still fits.
-constexpr int FL_DEP = 4;
 
 bool linear_kind(uint32_t kind) {
     switch (kind) {
@@ -1461,16 +1499,18 @@ int enqueue_jobs(const uq_linear_job* jobs, int count, hipStream_t s) {
         int threads = FL_WG;
         bool few = false;
         if (!rows_only) {
-            // Tiles per workgroup, from those that make one to four workgroups a
-            // CU: the fewest instructions that a CU runs one behind the other, the
-            // staging of x in every workgroup among them. One workgroup a CU (two
-            // waves per SIMD) leaves some of its time idle.
+            a.parts = plan_parts(lds, &lds);
             int64_t tiles = 0;
             for (int i = 0; i < jobs_here; i++)
                 if (!row_kind((uint32_t)a.job[i].kind)) tiles += (a.job[i].m + 15) / 16;
-            int64_t best = 0;
+            // Tiles per workgroup. Of a table: from those that make one to four
+            // workgroups a CU the fewest instructions that a CU runs one behind the
+            // other, the staging of x in every workgroup among them. One workgroup a
+            // CU (two waves per SIMD) leaves some of its time idle.
+            const int64_t alone = one ? single_wgs((uint32_t)a.job[0].kind, a.job[0].n, tiles, lds, cu) : 0;
+            int64_t best = one ? (tiles + alone - 1) / alone : 0;
             double least = 0.0;
-            for (int c = 0; c < 8; c++) {
+            for (int c = 0; c < 8 && !one; c++) {
                 const int64_t nt = (tiles + (c / 2 + 1) * cu - 1) / ((c / 2 + 1) * cu) + (c & 1);
                 int64_t wgs = 0;
                 double work = 0.0;
@@ -1492,13 +1532,10 @@ int enqueue_jobs(const uq_linear_job* jobs, int count, hipStream_t s) {
             for (int i = 0; i < jobs_here; i++) {
                 FJob& j = a.job[i];
                 j.wg0 = (int32_t)wg;
-                j.wgs = (int32_t)(row_kind((uint32_t)j.kind) ? std::min<int64_t>((j.m + 7) / 8, 4 * cu)
-                                                             : ((j.m + 15) / 16 + best - 1) / best);
+                j.wgs = (int32_t)(one ? alone : (row_kind((uint32_t)j.kind) ? std::min<int64_t>((j.m + 7) / 8, 4 * cu)
+                                                                            : ((j.m + 15) / 16 + best - 1) / best));
                 wg += j.wgs;
             }
-            a.parts.at = (int)((lds + 15) & ~(size_t)15);
-            a.parts.dep = a.parts.at <= 64 * 1024 ? FL_DEP : 1;
-            lds = (size_t)a.parts.at + 2 * 8 * 64 * FL_SEGS * (size_t)a.parts.dep;
         } else {
             // F32 / BF16: as many workgroups as fit on the chip at once; where
             // 512-thread ones cannot fill it, 256-thread ones, twice as many

@@ -30,10 +30,11 @@ def weight(kind, n, m):
 
 
 SHAPES = [(uq.KIND_Q8_0, n, m) for n, m in [(32, 1), (32, 9000), (96, 257), (992, 255), (1536, 4097), (1536, 40000),
-                                            (4096, 7000), (4128, 100), (8960, 3), (16352, 64), (16384, 1)]]
+                                            (4096, 7000), (4128, 100), (8960, 3), (16352, 64), (16384, 1),
+                                            (10240, 70), (10272, 70), (512, 98304), (512, 98320)]]
 SHAPES += [(k, n, m) for k in (uq.KIND_Q4_K, uq.KIND_Q3_K)
            for n, m in [(256, 1), (256, 33000), (768, 257), (1536, 4097), (1536, 140000), (4096, 20001), (8960, 100),
-                        (8960, 4000), (16384, 5)]]
+                        (8960, 4000), (16384, 5), (1024, 147456), (1024, 147488)]]
 
 
 @pytest.mark.parametrize("kind,n,m", SHAPES)

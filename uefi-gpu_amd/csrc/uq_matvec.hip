@@ -729,18 +729,26 @@ constexpr int TWO_LAUNCHES = 1;  // launch_kind's answer where x is better quant
 //   K 4096   g 256 6.4 -> 4.4   g 1024 7.7 -> 6.7     g 4000 13.7 -> 14.3
 //   K 8960   g 256 6.3 -> 5.7   g 512 7.0 -> 7.5      g 1024 8.4 -> 10.0
 //   K 16384  g 256 6.6 -> 6.8   g 512 8.6 -> 9.6
-// One launch won at every point below the line K (g + 1.5 CUs) = 29000 CUs and
-// lost or tied at all but a few above it.
-bool quant_pays(int64_t K, int64_t g) {
+// Below the line K (g + 1.5 CUs) = 29000 CUs one launch won, and lost or tied at all
+// but a few points above it, with two exceptions below it (graphs of 24 calls, whose
+// gaps are shorter than those above; two launches -> one, us):
+//   K-quants, g > 18 CUs: K 1024 g 4748 20.1 -> 21.4, g 4000 17.5 -> 17.3
+//   Q8_0, K <= 512, g > 24 CUs: K 512 g 8000 13.5 -> 14.5, g 6000 11.2 -> 11.0, where
+//     K 768 g 8000 gives 19.0 -> 17.7
+bool quant_pays(bool q8, int64_t K, int64_t g) {
     const int64_t cu = cu_count();
+    if (q8 ? K <= 512 && g > 24 * cu : g > 18 * cu) return false;
     return K * (2 * g + 3 * cu) <= 58000 * cu;
 }
 
 // The register kernel's one-launch form. Only Q8_0's 16-value units take it: the
-// superblock kinds leave the LDS kernels past K = MAX_XL, where two launches win.
+// superblock kinds leave the LDS kernels past K = MAX_XL, where two launches win, as
+// they do for Q8_0 past MAX_QX: with few rows K 8960 4.3 -> 4.1 us, 12288 4.7 -> 4.8,
+// 16384 5.0 -> 5.8 (Q4_K in LDS 6.3 -> 5.9).
+constexpr int MAX_QX = 10240;
 template <class KQ, int LPR, int NBL>
 const void* fused_kernel() {
-    if constexpr (KQ::UNIT < 64) return (const void*)k_matvec_f<KQ, LPR, NBL>;
+    if constexpr (KQ::UNIT < 64 && LPR * NBL * KQ::UNIT <= MAX_QX) return (const void*)k_matvec_f<KQ, LPR, NBL>;
     return nullptr;
 }
 
@@ -771,7 +779,7 @@ bool launch_t(const Weight& w, const Weight* w2, const int8_t* xq, const float* 
     int64_t g = m * cu;
     if (g > fit) g = nblk;
     if (g > w.m) g = w.m;
-    if (x && !quant_pays(w.n, g)) return false;
+    if (x && !quant_pays(KQ::UNIT < 64, w.n, g)) return false;
     const unsigned grid = (unsigned)g;
     const int64_t share = w.m / g;
     WArgs a{w.qs, w.d, w.sc}, b{nullptr, nullptr, nullptr};
@@ -801,7 +809,7 @@ int launch_sb(const Weight& w, const Weight* w2, const int8_t* xq, const float* 
     const int nthr = bpw * g.LB;
     const unsigned grid = (unsigned)((g.blocks + bpw - 1) / bpw);
     const size_t lds = sb_lds_bytes(g.S, nthr, w2 != nullptr);
-    if (x && !quant_pays(w.n, grid)) return TWO_LAUNCHES;
+    if (x && !quant_pays(false, w.n, grid)) return TWO_LAUNCHES;
     const SbArgs a{g.S, g.LB, g.RB};
     const uint8_t* q = (const uint8_t*)w.qs;
     if (x)

@@ -192,15 +192,23 @@ struct LayoutArgs {
     int32_t kind, block_bytes, blocks;  // blocks per row
     int32_t steps, bps;                 // steps per row, blocks per step
     int32_t rec[3];                     // bytes of a tile's step in each plane
+    int64_t dwords[3];                  // of each plane
     uint8_t* plane[3];
 };
 
-// Code of value e (0..31) of 32-value block sb of an IQ3_XXS superblock.
-__device__ __forceinline__ uint32_t iq3_code(const uint8_t* p, int sb, int e) {
+// Codes of values e .. e + 3 (e % 4 == 0) of 32-value block sb of an IQ3_XXS
+// superblock, one a byte.
+__device__ __forceinline__ uint32_t iq3_codes(const uint8_t* p, int sb, int e) {
     const uint32_t s7 = (rd32(p + 66 + 4 * sb) >> (7 * (e / 8))) & 127u;
-    const uint32_t neg = ((s7 | (uint32_t)(__popc(s7) & 1) << 7) >> (e % 8)) & 1u;
-    const uint32_t level = ((c_iq3_grid[p[2 + 8 * sb + e / 4]] >> (8 * (e % 4))) & 255u) >> 3;
-    return nibble_of(book_codes(), neg ? 7 - level : 8 + level);
+    const uint32_t neg = (s7 | (uint32_t)(__popc(s7) & 1) << 7) >> (e % 8);
+    const uint32_t levels = c_iq3_grid[p[2 + 8 * sb + e / 4]] >> 3;
+    uint32_t v = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint32_t level = (levels >> (8 * k)) & 7u;
+        v |= nibble_of(book_codes(), (neg >> k) & 1u ? 7 - level : 8 + level) << (8 * k);
+    }
+    return v;
 }
 
 // Byte `at` of a tile's step in plane pl: what the block's bytes p (of the
@@ -240,11 +248,7 @@ __device__ uint32_t plane_byte(const LayoutArgs& a, const uint8_t* src, int pl, 
             return (uint32_t)((int)((p[4 + sb / 2] >> (4 * (sb % 2))) & 15) + (int)(((rd16(p + 2) >> (2 * sb)) & 3) << 4) - 32) & 255u;
         }
     case KIND_IQ3_XXS:
-        if (pl == FL_BODY) {
-            const int sb = 4 * (o >> 4) + g;
-            return iq3_code(p, sb, o & 15) | iq3_code(p, sb, 16 + (o & 15)) << 4;
-        }
-        if (o >= 8) return p[o - 8];
+        if (o >= 8) return p[o - 8];  // (the body: k_layout_repack)
         return 2 * (p[66 + 4 * (2 * (o & 3) + (o >> 2)) + 3] >> 4) + 1;
     default:  // Q6_K
         if (pl == FL_BODY)
@@ -254,14 +258,26 @@ __device__ uint32_t plane_byte(const LayoutArgs& a, const uint8_t* src, int pl, 
     }
 }
 
-// One dword of a plane per thread; rows past the last and columns past n are zero.
-__global__ __launch_bounds__(FWG) void k_layout_repack(const uint8_t* __restrict__ src, LayoutArgs a, int pl, int64_t dwords) {
-    for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < dwords; i += (int64_t)gridDim.x * FWG) {
+// One dword of a plane per thread, the planes one behind the other; rows past the
+// last and columns past n are zero. The bytes of an IQ3_XXS body hold two codes
+// each and are made four at a time, as their grid words and signs are shared.
+__global__ __launch_bounds__(FWG) void k_layout_repack(const uint8_t* __restrict__ src, LayoutArgs a, int64_t total) {
+    for (int64_t j = (int64_t)blockIdx.x * FWG + threadIdx.x; j < total; j += (int64_t)gridDim.x * FWG) {
+        int64_t i = j;
+        int pl = 0;
+        while (i >= a.dwords[pl]) i -= a.dwords[pl++];
         const int64_t rec = 4 * i / a.rec[pl];
         const int at = (int)(4 * i - rec * a.rec[pl]);
         uint32_t v = 0;
+        if (a.kind == KIND_IQ3_XXS && pl == FL_BODY) {
+            const int64_t tile = rec / a.steps, row = 16 * tile + ((at >> 4) & 15);
+            const int sb = 4 * (at >> 10) + ((at >> 8) & 3);
+            const uint8_t* p = src + (row * a.blocks + (rec - tile * a.steps)) * a.block_bytes;
+            if (row < a.m) v = iq3_codes(p, sb, at & 15) | iq3_codes(p, sb, 16 + (at & 15)) << 4;
+        } else {
 #pragma unroll 1
-        for (int k = 0; k < 4; k++) v |= plane_byte(a, src, pl, rec, at + k) << (8 * k);
+            for (int k = 0; k < 4; k++) v |= plane_byte(a, src, pl, rec, at + k) << (8 * k);
+        }
         ((uint32_t*)a.plane[pl])[i] = v;
     }
 }
@@ -290,35 +306,6 @@ __device__ int source_byte(const LayoutArgs& a, int64_t row, int64_t b, int o) {
         }
         if (o < 8) return ((scale(2 * (o - 4)) + 32) & 15) | ((scale(2 * (o - 4) + 1) + 32) & 15) << 4;
         return (int)recode(book_places(), body(((o - 8) >> 4) & 3, 16 * ((o - 8) >> 6) + ((o - 8) & 15)));
-    case KIND_IQ3_XXS: {
-        if (o < 2) return a.plane[FL_ROW][rec * 160 + 128 + 2 * r + o];
-        // place in ascending order of value e of block sb: below 8 negative
-        auto place = [&](int sb, int e) {
-            return nibble_of(book_places(), (body(sb & 3, 16 * (sb >> 2) + (e & 15)) >> (4 * (e >> 4))) & 15u);
-        };
-        if (o < 66) {  // the grid index of four levels (the grid ascends)
-            const int sb = (o - 2) >> 3, e = 4 * ((o - 2) & 7);
-            uint32_t w = 0;
-            for (int k = 0; k < 4; k++) {
-                const uint32_t q = place(sb, e + k), level = q < 8 ? 7 - q : q - 8;
-                w |= (level == 7 ? 62u : 8 * level + 4) << (8 * k);
-            }
-            int lo = 0;
-            for (int step = 128; step; step >>= 1)
-                if (c_iq3_grid[lo + step] <= w) lo += step;
-            return c_iq3_grid[lo] == w ? lo : -1;
-        }
-        const int sb = (o - 66) >> 2;
-        uint32_t aux = (uint32_t)(scale(sb) >> 1) << 28;
-        bool even = (scale(sb) & 1) != 0;
-        for (int k = 0; k < 4; k++) {
-            uint32_t neg = 0;
-            for (int e = 0; e < 8; e++) neg |= (place(sb, 8 * k + e) < 8 ? 1u : 0u) << e;
-            even = even && (__popc(neg) & 1) == 0;
-            aux |= (neg & 127u) << (7 * k);
-        }
-        return even ? (int)((aux >> (8 * ((o - 66) & 3))) & 255u) : -1;
-    }
     default: {  // Q6_K
         if (o < 128) return (int)body(2 * (o >> 6) + ((o >> 4) & 1), 16 * ((o >> 5) & 1) + (o & 15));
         if (o < 192) return (int)body(2 * ((o - 128) >> 5) + ((o >> 4) & 1), 32 + (o & 15));
@@ -337,6 +324,49 @@ __global__ __launch_bounds__(FWG) void k_layout_verify(const uint8_t* __restrict
     for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < total; i += (int64_t)gridDim.x * FWG) {
         const int64_t blk = i / a.block_bytes, row = blk / a.blocks;
         miss += source_byte(a, row, blk - row * a.blocks, (int)(i - blk * a.block_bytes)) != (int)src[i];
+    }
+    if (miss) atomicAdd(bad, miss);
+}
+
+// An IQ3_XXS superblock from its planes, a 32-value block per thread: the eight grid
+// words (the grid's entries are distinct, so one names its index), the signs with
+// their parity, the scale, and with block 0 the two bytes of d. Byte by byte, with
+// a search of the grid, 50000 x 2560 took 0.5 ms longer to upload.
+__global__ __launch_bounds__(FWG) void k_iq3_verify(const uint8_t* __restrict__ src, LayoutArgs a, int64_t total,
+                                                    unsigned* bad) {
+    unsigned miss = 0;
+    for (int64_t i = (int64_t)blockIdx.x * FWG + threadIdx.x; i < total; i += (int64_t)gridDim.x * FWG) {
+        const int64_t blk = i >> 3, row = blk / a.blocks, rec = (row >> 4) * a.steps + (blk - row * a.blocks);
+        const int sb = (int)(i & 7), r = (int)(row & 15);
+        const uint8_t* p = src + blk * a.block_bytes;
+        const uint8_t* rr = a.plane[FL_ROW] + rec * a.rec[FL_ROW];
+        const uint4 b = *(const uint4*)(a.plane[FL_BODY] + rec * a.rec[FL_BODY] + 1024 * (sb >> 2) + 16 * (16 * (sb & 3) + r));
+        const uint32_t v[4] = {b.x, b.y, b.z, b.w};
+        uint32_t signs = 0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                // place in ascending order: below 8 negative
+                const uint32_t place = nibble_of(book_places(), (v[q & 3] >> (8 * k + 4 * (q >> 2))) & 15u);
+                const uint32_t level = place < 8 ? 7 - place : place - 8;
+                w |= (level == 7 ? 62u : 8 * level + 4) << (8 * k);
+                signs |= (place < 8 ? 1u : 0u) << (4 * q + k);
+            }
+            miss += c_iq3_grid[p[2 + 8 * sb + q]] != w;
+        }
+        const int sc = (int)(int8_t)rr[8 * r + 4 * (sb & 1) + (sb >> 1)];
+        uint32_t aux = (uint32_t)(sc >> 1) << 28;
+        miss += (sc & 1) == 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t neg = (signs >> (8 * k)) & 255u;
+            miss += (unsigned)__popc(neg) & 1u;
+            aux |= (neg & 127u) << (7 * k);
+        }
+        miss += aux != rd32(p + 66 + 4 * sb);
+        if (sb == 0) miss += rd16(rr + 128 + 2 * r) != rd16(p);
     }
     if (miss) atomicAdd(bad, miss);
 }
@@ -1434,12 +1464,15 @@ void launch_layout(uint32_t kind, const uint8_t* src, int64_t n, int64_t m, cons
     for (int i = 0; i < 3; i++) {
         a.rec[i] = L.rec[i];
         a.plane[i] = planes[i];
+        a.dwords[i] = (int64_t)frontier_plane_bytes(L, i, n, m) / 4;
     }
-    for (int i = 0; i < 3; i++)
-        if (L.rec[i]) {
-            const int64_t dwords = (int64_t)frontier_plane_bytes(L, i, n, m) / 4;
-            hipLaunchKernelGGL(k_layout_repack, dim3(grid_blocks(dwords)), dim3(FWG), 0, s, src, a, i, dwords);
-        }
+    const int64_t dwords = a.dwords[0] + a.dwords[1] + a.dwords[2];
+    hipLaunchKernelGGL(k_layout_repack, dim3(grid_blocks(dwords)), dim3(FWG), 0, s, src, a, dwords);
+    if (kind == KIND_IQ3_XXS) {
+        const int64_t subs = m * a.blocks * 8;
+        hipLaunchKernelGGL(k_iq3_verify, dim3(grid_blocks(subs)), dim3(FWG), 0, s, src, a, subs, bad);
+        return;
+    }
     hipLaunchKernelGGL(k_layout_verify, dim3(grid_blocks(total)), dim3(FWG), 0, s, src, a, total, bad);
 }
 

@@ -96,7 +96,7 @@ struct FrontierLayout {
 bool frontier_layout(uint32_t kind, FrontierLayout& L);
 size_t frontier_plane_bytes(const FrontierLayout& L, int plane, int64_t n, int64_t m);
 // Repacks GGUF rows into the planes, then rebuilds every GGUF byte from them and
-// adds the number of differing ones to *bad.
+// adds the number of differing ones (IQ3_XXS: pieces of a block) to *bad.
 void launch_layout(uint32_t kind, const uint8_t* src, int64_t n, int64_t m, const FrontierLayout& L,
                    uint8_t* const planes[3], unsigned* bad, hipStream_t s);
 

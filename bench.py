@@ -394,8 +394,8 @@ def frontier_moe_bench(tokens=32, reps=3, experts=256, top_k=10, dim=2560, ff=64
     nbuf = dim + experts + 23 * ff + 11 * ff + 11 * dim
     buf = ctypes.c_void_p()
     uq._check(L.uq_dev_alloc(4 * nbuf, ctypes.byref(buf)))
-    uq._check(L.uq_memcpy_h2d(buf, np.ascontiguousarray(rng.normal(0, 1, nbuf).astype(np.float32)).ctypes.data,
-                              4 * nbuf))
+    init = rng.normal(0, 1, nbuf).astype(np.float32)  # (named: the copy below reads it by address)
+    uq._check(L.uq_memcpy_h2d(buf, init.ctypes.data, init.nbytes))
     at = lambda off: buf.value + 4 * off
     x, sc = at(0), at(dim)
     proj = [at(dim + experts + i * ff) for i in range(23)]

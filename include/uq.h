@@ -74,7 +74,11 @@ typedef struct uq_weight* uq_weight_t;
  * IQ4_XS for the fp32-activation reader (F32/BF16: n % 8 == 0). */
 int uq_weight_upload(uint32_t kind, int64_t n, int64_t m, const void* gguf, size_t bytes, uq_weight_t* out);
 int uq_weight_free(uq_weight_t w);
-/* Device bytes held by the weight (repacked planes). */
+/* Device bytes held by the weight (repacked planes). Q8_0, Q6_K and IQ4_NL take
+ * their GGUF bytes, IQ4_XS 138 per 256 values for 136, IQ3_XXS 138 for 98 (its
+ * codes are written out); Q6_K and the IQ kinds are laid out in tiles of 16 rows
+ * (IQ4_NL: by 128 columns), so that a weight of one row takes the bytes of 16.
+ * Each plane is padded to 256 bytes. */
 int64_t uq_weight_bytes(uq_weight_t w);
 
 /* ---------------------------------------------------------------- linears */
@@ -98,12 +102,14 @@ int uq_matvec_q_dev(uq_weight_t w, const int8_t* xq, const float* xs, float* y, 
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): uq_matvec on device pointers, x (n floats) -> y (m
- * floats) on `stream` (NULL: library stream), without synchronizing. The
- * quantized activation goes to a static device scratch of the library
- * (n <= 16384, else UQ_ERR_SHAPE); the call allocates and frees nothing. Every
- * call on one GPU shares that scratch: calls that overlap on one GPU (other
- * streams, other threads) race. Output equals uq_matvec's bit for bit; x is
- * not checked for non-finite values. */
+ * floats) on `stream` (NULL: library stream), without synchronizing. Where the
+ * quantized activation is a launch of its own it goes to a static device scratch
+ * of the library (n <= 16384, else UQ_ERR_SHAPE); where one launch quantizes and
+ * multiplies, each workgroup keeps it in LDS. Which form runs depends on kind,
+ * sizes and the alignment and place of x, so count every call on one GPU as using
+ * that scratch: calls that overlap (other streams, other threads) race. The call
+ * allocates and frees nothing. Output equals uq_matvec's bit for bit; x is not
+ * checked for non-finite values. */
 int uq_matvec_static(uq_weight_t w, const float* x, float* y, void* stream);
 /* gateup_dp4a (gpu_dp4a.cu:60-64): out[r] = silu(gate_r . x) * (up_r . x). */
 int uq_gateup_q_dev(uq_weight_t gate, uq_weight_t up, const int8_t* xq, const float* xs, float* out, void* stream);

@@ -81,9 +81,10 @@ def test_linear_random_shapes(gpu, kind, n, m):
 
 
 def wide_range_x(n, seed):
-    """x whose 32-blocks exercise the exact-integer staging: zeros, denormals,
-    a 2^20 range (double path), 1e30 beside 1e-30 (double path), small values
-    with zero low bits beside a large one (integer path), -0.0, ordinary."""
+    """x for the exact-integer staging, which takes groups of 256 values: in the
+    first group zeros, denormals and ordinary values, all more than 2^38 below the
+    1e30 among them and so in the double path (but for the zeros and -0.0); the
+    groups behind it are ordinary."""
     rng = np.random.default_rng(seed)
     x = rng.normal(0, 1, n).astype(np.float32)
     x[0:32] = 0

@@ -23,14 +23,19 @@
 // Bound and choices (MI355X, HIP events over back-to-back launches, before ->
 // after, "before" being five v_dot4 digit planes with 8-16 lanes a row):
 //  * digits on the matrix core: v_dot4 needed 1.25 instructions and 5 bytes of
-//    LDS per weight; v_mfma_i32_16x16x64_i8 takes eight digits of 1,024 weights
-//    in one instruction and 0.25 bytes of LDS per weight. What is left on the
-//    VALU is the unpacking of the codes (IQ4/IQ3: 88 of 150 instructions a step
-//    of 16 rows x 256 columns), which bounds large IQ weights; Q6_K and Q8_0
-//    reach 5.4 and 4.7 TB/s of a 7.0 TB/s streaming read.
-//  * 52000 x 2560: Q6_K 38.8 -> 22.2 us, IQ3_XXS 32.8 -> 18.4, IQ4_NL 30.0 ->
-//    22.0, IQ4_XS 31.2 -> 18.4, Q8_0 30.8 -> 30.9. 256 x 16384: Q6_K 52.6 ->
-//    13.4, Q8_0 28.4 -> 17.6. 640 x 2560: IQ3_XXS 10.2 -> 4.8.
+//    LDS per weight. v_mfma_i32_16x16x64_i8 takes all eight digits, of 1,024
+//    weights in Q8_0 and of 512 in the other kinds, whose scale groups lie so that
+//    each operand of codes goes out twice; an instruction reads 1 KB of digits, 1
+//    and 2 bytes per weight, half or a quarter of it other than the zeros of a
+//    foreign slice. What is left on the VALU is the unpacking of the codes (IQ4_XS
+//    and IQ3_XXS: 122 instructions beside 8 products a step of 16 rows x 256
+//    columns, 88 of them the code book), which bounds large IQ weights; Q6_K and
+//    Q8_0 reach 5.9 and 5.3 TB/s at 151936 x 2560, of a 7.0 TB/s streaming read.
+//  * 52000 x 2560: Q6_K 38.0 -> 21.4 us, IQ3_XXS 33.0 -> 17.2, IQ4_NL 31.0 ->
+//    20.5, IQ4_XS 32.6 -> 17.1, Q8_0 30.0 -> 29.9. 256 x 16384: Q6_K 59.3 ->
+//    13.6, Q8_0 34.4 -> 18.3. 640 x 2560: IQ3_XXS 10.2 -> 4.8. Q8_0 of 2560
+//    columns and 70000 rows or more is 3 to 5% slower (37.0 -> 38.8 us), of 2048
+//    or 4096 columns 6 to 12% faster.
 //  * tiles of 16 rows are laid out at upload in the order in which a wave reads
 //    them (whole kilobytes per load instruction); Q8_0 shares the int8 matvec's
 //    row planes.
@@ -545,10 +550,14 @@ __device__ __forceinline__ void to_slices(uint32_t v, uint32_t (&out)[2]) {
 // A wave walks a tile of 16 rows in steps of VPS columns; U is what a lane
 // loads for one step, NB how many steps are in flight. Two pay where the bytes
 // per instruction are many (Q8_0 and Q6_K, 52000 x 2560: 35.8 -> 30.9 us, 25.2 ->
-// 22.2); elsewhere, and for short waves (one_kernel), the smaller code of one
-// does (IQ4_XS 3001 x 2560: 5.10 -> 4.85 us; three or four are slower still). step() adds the step's products to the lane's four digit
-// sums; chunk() gives 16 codes, their first column and their scale for the
-// products of a wide group in double.
+// 22.2; Q8_0 with three or four within 4% of it from n 2048 on, slower below); for
+// short waves (one_kernel) the smaller code of one does. The IQ kinds have one: two
+// make IQ4_XS and IQ3_XXS 3 to 15% slower to n 1024 (151936 rows 3% faster) and 9%
+// slower to 4% faster at 2560, but 15% faster at n 8192 from 13000 rows on (IQ4_NL
+// 24%; at 2560 1% slower to 9% faster), where a CU holds
+// one workgroup. step() adds the step's products to the lane's four digit sums;
+// chunk() gives 16 codes and their scale, column() their first column, for the
+// products that run in double.
 
 // 16 codes of a 32-value block of nibbles through a code book: the low nibbles
 // are its values 0..15, the high ones 16..31.
@@ -1031,6 +1040,9 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         // without one left out. 49344 x 2560 with one such value in x / one in
         // each group, against one wave summing all products of a group with one:
         // Q8_0 65.6 -> 30.6 us / 254 -> 41.7, IQ3_XXS 43.6 -> 21.6 / 214 -> 33.3.
+        // Where x is full of them it costs more: with one value in twenty / in two
+        // Q8_0 82 / 82 us, Q6_K 68 / 68, IQ4_XS 54 / 56 (65 / 75, 60 / 54 and 64 / 73
+        // with 32-value blocks of a range over 2^14 in double).
         int base = 0, buffer = 0;
         auto flush = [&]() {
             const int to = base + dep < count ? base + dep : count;
@@ -1185,11 +1197,6 @@ __device__ void job_rows(const FJob& j, int wgi, int wgc, const XStage& xs) {
     }
 }
 
-template <class T>
-constexpr int rows_per_wave() {
-    return 64 / T::LPR;
-}
-
 // Up to MAX_JOBS jobs per launch, passed by value in the kernel arguments
 // (no device table to copy before the launch); longer tables take several
 // launches, each row computed the same way.
@@ -1262,9 +1269,9 @@ __device__ __forceinline__ void run_job(const FJob& j, int wgi, const Parts& par
 }
 
 // One job, its record in the first lines of the arguments. Four waves per SIMD,
-// two workgroups of a CU at work, for the tiled kinds. The row kinds stream their
-// rows at whatever their registers allow: with the same bound the compiler gave F32
-// 88 registers for 96, and 100000 x 256 took 34.6 us for 30.5.
+// two workgroups of a CU at work, for the tiled kinds. The row kinds use fewer
+// registers by themselves, but under the same bound the compiler scheduled F32 with
+// more waits for all loads in flight, and 100000 x 256 took 34.6 us for 30.5.
 struct OneJob {
     Parts parts;
     FJob job;

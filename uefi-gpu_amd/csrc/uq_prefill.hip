@@ -889,6 +889,12 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t s) {
         // a layer at K = 8960: 96 workgroups 26.7 -> 18.1 us, 384 26.2 -> 23.7,
         // 768 31.0 -> 39.4; at K = 1536: 96 6.3 -> 5.4 us, 128 7.4 -> 6.4, 256
         // 7.5 -> 6.8, 512 8.2 -> 8.7 (12 stages are too few to pay for the fill).
+        // With more than one workgroup per CU the line was drawn by whole prompts
+        // of 140 to 320 tokens, 8 layers, 4 -> 8 stages: q|k|v and o at K 1536 +2.2%,
+        // down at K 3072 nothing beside that, 4096 -0.9%, 6144 -2.3%, 8960 -2.0%. A
+        // single GEMM over and over, its weights in the caches, is 3 to 5% slower
+        // with 8 stages at K 512 and 1536 (no layer runs so), 2 to 10% faster from
+        // K 3072 on.
         if (wgs <= (a.k >= 4096 ? 2 : 1) * cu) UQ_GEMM(false, 1, 8);
         else UQ_GEMM(false, 1, 4);
     } else {

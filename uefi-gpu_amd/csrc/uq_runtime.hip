@@ -164,7 +164,11 @@ void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
 // Waits for the work on the library stream: a last launch stores a number to
 // pinned memory and the host watches for it, which two launches and
 // hipStreamSynchronize take 14.1-15.5 us for and this 10.7-12.1. The watch is
-// bounded; hipStreamSynchronize then waits, and reports what failed.
+// bounded; hipStreamSynchronize then waits, and reports what failed. Outputs that
+// earlier launches stored to the pinned buffer are visible once the number is: the
+// stream runs its launches one behind the other, the buffer is fine-grained host
+// memory (hipHostMallocDefault), which no GPU cache keeps back, and the number is a
+// release at system scope that the host reads with an acquire.
 hipError_t wait_host() {
     const uint32_t want = ++g_ctx.waits;
     hipLaunchKernelGGL(k_flag, dim3(1), dim3(1), 0, g_ctx.stream, g_ctx.flag, want);

@@ -497,7 +497,7 @@ __device__ __forceinline__ uint64_t stage_x(const float* __restrict__ x, int n, 
             for (int k = 0; k < 4; k++) d[4 + k] = t[k];
         }
         const uint64_t out = __builtin_amdgcn_ballot_w64(!ok);
-        if (out) {
+        if (__builtin_expect(out != 0, 0)) {
             wide |= 1ull << grp;
             if (lane == 0) far[grp] = out;
 #pragma unroll
@@ -1000,7 +1000,10 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
         return __builtin_fma(t, 256.0, acc[0]) * half;
     };
     Place p(wave, S);
-    if (xs.wide == 0) {
+    // (expected, so that the double branches lie behind the code that runs: a call of
+    // a few microseconds is some 1% longer where it fetches instructions across them,
+    // IQ4_XS 3001 x 2560 4.85 us for 4.79)
+    if (__builtin_expect(xs.wide == 0, 1)) {
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
         int base = 0, buffer = 0;
         // once the wave is past them, the workgroup sums the tiles from `base` on
@@ -1069,7 +1072,7 @@ __device__ __forceinline__ void job_tiles(const FJob& j, int wgi, int dep, doubl
 #pragma unroll 1
         while (base < count) flush();
     }
-    if (__builtin_amdgcn_ballot_w64(again) == 0) return;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(again) == 0, 1)) return;
 #pragma unroll 1
     for (int i = 0; i < count; i++) {
         if (((i % dep) & (FL_SEGS - 1)) != wave) continue;
